@@ -265,6 +265,11 @@ typedef struct sf_camera {
  * angle |dot(normalize(cam - p), n)| (bubble.wgsl:491-494), contracted with
  * cmf[81][3] on 16-bit MFMA with FP32 accumulation:
  *   rgb[c][cell] = (1/81) sum_k I_k cmf[k][c].
+ * On grids of 2^20 cells and more with films up to about 2 um the sum is
+ * evaluated, in the AUTO format, as a cosine series in the phase (FP32, each
+ * channel within 2e-5 sum_k |cmf[k][c]| / 81 of the sum over the
+ * wavelengths); the contraction then serves cells seen within about 3
+ * degrees of grazing.
  * Operand format (sf_spectral_set_operand): by default FP16 when its
  * rounding of the reflectance moves no channel by more than 2.5e-4
  * (2^-18 sum_k |cmf[k][c]|) and the curves fit FP16, else a BF16 hi/lo
@@ -321,7 +326,7 @@ int sf_spectral_kernel_timing(sf_drainage* ctx, int32_t enable, double* avg_ms,
 #define SF_SPECTRAL_OPERAND_BF16_PAIR 1
 #define SF_SPECTRAL_OPERAND_FP16 2
 int sf_spectral_set_operand(sf_drainage* ctx, int32_t kind);
-/* Operand format the next spectral call uses with the curves last given
+/* Operand format of the next spectral call's contraction with the curves last given
  * (SF_SPECTRAL_OPERAND_BF16_PAIR or _FP16; AUTO before any curves). */
 int sf_spectral_get_operand(sf_drainage* ctx, int32_t* kind);
 

@@ -379,6 +379,13 @@ void Drainage::update_fixed_pole_mass() {
 // writes (the poles, and Γ when it is frozen) hold the same values in both.
 void Drainage::upload(const float* h_hi, const float* h_lo, const float* gam) {
     if (h_hi) {
+        // independent maxima, so that the loop vectorises
+        float mx[32] = {0.f};
+        size_t k0 = 0;
+        for (; k0 + 32 <= n; k0 += 32)
+            for (int j = 0; j < 32; ++j) mx[j] = h_hi[k0 + j] > mx[j] ? h_hi[k0 + j] : mx[j];
+        for (; k0 < n; ++k0) mx[0] = std::max(mx[0], h_hi[k0]);
+        h_max = *std::max_element(mx, mx + 32);
         for (int k = 0; k < 2; ++k) {
             SF_HIP(hipMemcpyAsync(hi[k], h_hi, n * sizeof(float), hipMemcpyHostToDevice, stream));
             SF_HIP(hipMemcpyAsync(lo[k], h_lo, n * sizeof(float), hipMemcpyHostToDevice, stream));
@@ -398,6 +405,7 @@ void Drainage::upload(const float* h_hi, const float* h_lo, const float* gam) {
 void Drainage::fill(double h0, double gamma0) {
     const float h_hi = static_cast<float>(h0);
     const float h_lo = static_cast<float>(h0 - static_cast<double>(h_hi));
+    h_max = h0;
     for (int k = 0; k < 2; ++k) {
         hipLaunchKernelGGL(fill_kernel, dim3(cdiv(n, 256)), dim3(256), 0, stream, hi[k], n, h_hi);
         hipLaunchKernelGGL(fill_kernel, dim3(cdiv(n, 256)), dim3(256), 0, stream, lo[k], n, h_lo);

@@ -84,6 +84,7 @@ struct Drainage {
     float2* hpole_mid[2] = {nullptr, nullptr};
     int cur_mid = 0;
     bool poles_virtual = false;   // pole rows are held as ring partials
+    double h_max = 0.0;           // largest thickness last uploaded or filled, m (a kernel choice, not a bound)
     RowF* rows = nullptr;
     RowD* rowd = nullptr;
     bool tables_dirty = true;
@@ -119,6 +120,11 @@ struct Drainage {
     float* rgb = nullptr;
     float* caustic = nullptr;       // caustic-intensity map (caustics.hip), allocated on first use
     float* cmf_dev = nullptr;       // colour curves as MFMA B fragments
+    float* cmf_series = nullptr;    // their cosine-series table (spectral_series_kernel), behind the fragments
+    unsigned* spec_list = nullptr;  // cells of a near-grazing view (spectral_list_kernel), then their count; behind spec_view
+    float cmf_host[243];            // the curves laid out in both, valid when cmf_valid
+    bool cmf_valid = false, series_valid = false;
+    float cmf_mean[3] = {0.f, 0.f, 0.f};   // mean over the wavelengths of each curve
     // Per operand format (0: BF16 hi/lo pair, 1: FP16): sum over the 81
     // wavelengths of each curve as the MFMA sees it, and whether the curves
     // need their lo fragments.
@@ -129,7 +135,7 @@ struct Drainage {
     int cmf_skip = 0;               // trailing wavelength slots the spectral pass leaves out
     int spec_operand = 0;           // SF_SPECTRAL_OPERAND_*
     float4* spec_rows = nullptr;
-    float2* spec_view = nullptr;    // per-cell (F, cos theta_t) of spec_view_key's camera and index
+    float2* spec_view = nullptr;    // per-cell (q, opd per thickness) of spec_view_key's camera and index
     float spec_view_key[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     bool spec_view_valid = false;
     float2* spec_cols = nullptr;

@@ -6,8 +6,11 @@
 //                       in FP32 (3 wavelengths, gamma 1/2.2): 1-D/2-D LUTs,
 //                       per-point colour, intensity and intermediate terms
 //   spectral_kernel     81-wavelength Airy/Fresnel reflectance at every grid
-//                       cell's view angle, contracted with cmf[81][3] on BF16
-//                       MFMA (v_mfma_f32_16x16x32_bf16) with FP32 accumulation
+//                       cell's view angle, contracted with cmf[81][3] on 16-bit
+//                       MFMA (v_mfma_f32_16x16x32) with FP32 accumulation
+//   spectral_series_kernel, spectral_list_kernel
+//                       the same as a cosine series in the phase, for large
+//                       grids (the default there)
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -308,9 +311,10 @@ struct SpecArgs {
     // from hpole, as materialize_poles_kernel would write it.
     const float2* hpole;
     int pole_virtual, nt, ntiles;
-    // Per-cell (F, cos theta_t) of the current camera and film index; the
+    // Per-cell (q, optical path per thickness) of the current camera and film
+    // index: F = 4 q / (1 - q)^2, opd = h view.y in nm for h in m.  The
     // geometry is fixed while they are, so spectral_view_kernel computes it
-    // once; spectral_kernel reads it from here.
+    // once.
     const float2* view;
 };
 
@@ -328,8 +332,10 @@ __device__ inline void spec_cell_ij(const SpecArgs& a, size_t cc, float inv_np, 
     if (j >= a.np) { ++i; j -= a.np; }
 }
 
-// Coefficient of finesse F and cos theta_t of cell (i, j) at its view angle.
-__device__ inline void spec_view_terms(const SpecArgs& a, int i, int j, float& Fc, float& cos_t_out) {
+// q and cos theta_t of cell (i, j) at its view angle: q is the reflectance R
+// where F = 4 R / (1 - R)^2 is not clamped (interference_lut.rs:66-70 keeps
+// 1 - R at 1e-3 or more), else the root of 4 q / (1 - q)^2 = F.
+__device__ inline void spec_view_terms(const SpecArgs& a, int i, int j, float& q, float& cos_t_out) {
     const float4 rw = a.rows[i];
     const float2 cl = a.cols[j];
     // View angle |dot(normalize(cam - p), n)|, p = R n (bubble.wgsl:491-494).
@@ -344,22 +350,30 @@ __device__ inline void spec_view_terms(const SpecArgs& a, int i, int j, float& F
     const float rs = (cos_i - a.n_film * cos_t) * __builtin_amdgcn_rcpf(fmaxf(cos_i + a.n_film * cos_t, 1e-4f));
     const float rp = (a.n_film * cos_i - cos_t) * __builtin_amdgcn_rcpf(fmaxf(a.n_film * cos_i + cos_t, 1e-4f));
     const float R = (rs * rs + rp * rp) * 0.5f;
-    const float omr = fmaxf(1.f - R, 1e-3f);
-    Fc = 4.f * R * __builtin_amdgcn_rcpf(omr * omr);
+    q = R;
+    if (1.f - R < 1e-3f) {
+        const float s = sqrtf(1.f + 4e6f * R);
+        q = (s - 1.f) / (s + 1.f);
+    }
     cos_t_out = cos_t;
+}
+
+// Coefficient of finesse of a cell's q.
+__device__ inline float spec_finesse(float q) {
+    const float d = 1.f - q;
+    return 4.f * q * __builtin_amdgcn_rcpf(d * d);
 }
 
 // Per-cell terms of the Airy sum: coefficient of finesse F and optical path
 // difference opc (nm) of cell cc at its view angle, from the view table
-// a.view (F, cos theta_t per cell) and the film state.  last_row is the
-// index of the first cell of row nt - 1.
+// a.view and the film state.  last_row is the index of the first cell of
+// row nt - 1.
 __device__ inline void spec_cell_terms(const SpecArgs& a, size_t cc, size_t last_row, float& Fc, float& opc) {
     // Streaming load: this VALU-bound pass has bandwidth to spare, and the
     // film state should keep the cache.
     typedef float f2v __attribute__((ext_vector_type(2)));
     const f2v v = __builtin_nontemporal_load(reinterpret_cast<const f2v*>(a.view) + cc);
-    Fc = v.x;
-    const float cos_t = v.y;
+    Fc = spec_finesse(v.x);
     const bool top = cc < static_cast<size_t>(a.np);
     float h;
     if (a.pole_virtual && (top || cc >= last_row)) {
@@ -368,8 +382,7 @@ __device__ inline void spec_cell_terms(const SpecArgs& a, size_t cc, size_t last
     } else {
         h = a.hi[cc] + a.lo[cc];
     }
-    const float d_nm = h * 1e9f;
-    opc = 2.f * a.n_film * d_nm * cos_t;
+    opc = h * v.y;
 }
 
 // r' = r / 81 of one slot from its phase x in revolutions.  FAST:
@@ -561,15 +574,329 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
     }
 }
 
-__global__ __launch_bounds__(256) void spectral_view_kernel(const SpecArgs a, float2* __restrict__ out) {
-    const size_t cc = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x;
-    if (cc >= a.n) return;
-    int i, j;
-    spec_cell_ij(a, cc, 1.f / static_cast<float>(a.np), i, j);
-    float F, cos_t;
-    spec_view_terms(a, i, j, F, cos_t);
-    out[cc] = make_float2(F, cos_t);
+
+// The wavelength sum of the listed cells (spectral_view_kernel's: the view
+// so close to grazing that their series is long), 64 to a wave and batch,
+// every wave's next batch loaded ahead of its use.  Always the square form.
+template <bool F16, int SKIP>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) void spectral_list_kernel(
+    const SpecArgs a, const unsigned* __restrict__ list, const unsigned* __restrict__ count_dev) {
+    const int lane = threadIdx.x & 63, m = lane & 15, q = lane >> 4;
+    const unsigned count = *count_dev;
+    const unsigned step = gridDim.x * 4 * 64;
+    unsigned b = __builtin_amdgcn_readfirstlane((blockIdx.x * 4 + (threadIdx.x >> 6)) * 64);
+    if (b >= count) return;
+    unsigned cell = list[min(b + lane, count - 1)];
+    u32x2 pa[kSpecPhase];
+#pragma unroll
+    for (int e = 0; e < kSpecPhase; ++e) pa[e] = a.pfrag[e * 64 + lane];
+    const float u20 = a.ulam[4 * (kSpecSlots - 1) + q];
+    u32x4 bh[kSpecMfma], bl[kSpecMfma];
+#pragma unroll
+    for (int t = 0; t < kSpecMfma; ++t) {
+        bh[t] = a.bfrag[t * 64 + lane];
+        bl[t] = a.bfrag[(kSpecMfma + t) * 64 + lane];
+    }
+    const bool b_lo = a.b_lo != 0;
+    const float S = m == 0 ? a.s0 : (m == 1 ? a.s1 : a.s2);
+    const size_t last_row = static_cast<size_t>(a.nt - 1) * static_cast<size_t>(a.np);
+    float* plane = a.rgb + static_cast<size_t>(m < 3 ? m : 0) * a.n;
+    float Fc, opc;
+    spec_cell_terms(a, cell, last_row, Fc, opc);
+    while (b < count) {
+        const unsigned here = cell;
+        const int left = static_cast<int>(min(64u, count - b));
+        const float Bc = 81.f * Fc, Pc = opc;
+        b += step;
+        if (b < count) {
+            cell = list[min(b + lane, count - 1)];
+            spec_cell_terms(a, cell, last_row, Fc, opc);
+        }
+        const PhaseParts pp = phase_parts(Pc);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            if (16 * g >= left) break;
+            const int src = 16 * g + m;
+            u32x2 bop;
+            bop[0] = lane_read_u(pp.x0, src);
+            bop[1] = lane_read_u(pp.x1, src);
+            v4f acc = v4f{S, S, S, S};
+            spec_group<false, F16, SKIP>(pa, bop, u20, bh, bl, b_lo, lane_read(Pc, src), 81.f, lane_read(Bc, src), acc);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int k = 16 * g + 4 * q + v;
+                const unsigned to = lane_read_u(here, k);
+                if (m < 3 && k < left) plane[to] = acc[v];
+            }
+        }
+    }
 }
+
+// ---------------------------------------------------------------------------
+// The same sum as a cosine series in the phase.
+//
+// r = 1 / (1 + F cos^2(d / 2)), d = 2 pi opd / lambda, is the periodic function
+//   r = K [1 + 2 sum_{n >= 1} (-q)^n cos(n d)],
+//   s = sqrt(1 + F), K = 1 / s, q = (s - 1) / (s + 1)
+// (the Fourier series of 1 / (a + b cos d); with F = 4 R / (1 - R)^2, q is R),
+// so the sum over the wavelengths moves into three functions of one variable,
+//   G_c(y) = sum_k cmf[k][c] cos(2 pi y / lambda_k),
+//   rgb_c = S_c (1 - K) / 81 - (2 K / 81) sum_n (-q)^n G_c(n opd),
+// which depend on the curves alone.  They are tabulated once per set of
+// curves as cubics on intervals of kSerStep nm (interpolation at the four
+// Chebyshev points: error at most (2 pi kSerStep / lambda)^4 / 3072 of each
+// wavelength's share, 2.6e-5 at 380 nm, 6e-6 at 550 nm, times 2 q / (1 + q)), and a cell costs N table lookups
+// instead of 76-81 cosines and reciprocals.
+//
+// N: the terms after N sum to at most (S_c / 81) 2 q^(N+1), S_c = sum |cmf|, so
+// q^(N+1) <= kSerEps keeps them within 1.6e-5 S_c / 81 (2 terms at normal
+// incidence on a soap film, q = 0.02; 8 at q = 0.25).  Cells with q past
+// kSerMaxQ need more terms than the wavelength sum is worth (a view within 3
+// degrees of grazing, 8 % of a 2048 x 4096 grid); they are a matter of the
+// camera alone, so spectral_view_kernel lists them and spectral_list_kernel
+// takes the sum over the wavelengths for them.  Cells whose terms leave the
+// table (thick films) take that sum in place (series_direct).
+//
+// 2048 x 4096: 78 us (series 50, listed cells 23, the launches between them
+// 5) against 140 us for the wavelength sum everywhere (spectral_kernel); the
+// largest RGB error 2.5e-5 against 4.5e-5.  Of the series' 50 us, 43 are what
+// its 28 B per cell take with no term evaluated (5.4 TB/s); the rest is VALU
+// issue, 19 instructions per term.  The list runs a wavelength sum per cell
+// at a fifth of spectral_kernel's rate: scattered cells, two batches a wave.
+constexpr float kSerStep = 32.f;      // nm per table interval
+constexpr int kSerNodes = 1024;       // intervals of the table (48 KB of LDS)
+constexpr float kSerEps = 8e-6f;      // q^n below which a term is left out
+constexpr float kSerLog2 = -16.93f;   // log2 kSerEps
+constexpr int kSerThreads = 1024;
+constexpr size_t kSerWaves = kSerThreads / 64;
+constexpr size_t kSerBlocks = 512;
+constexpr unsigned kSerSkew = 97;
+// Smallest grid: two launches and the table's copy into LDS cost more than
+// they save on smaller ones (512 x 1024: 17.5 us against 12.8; 1024 x 2048:
+// 29.4 against 39.8).
+constexpr size_t kSerMinCells = size_t{1} << 20;
+// Thickest film, as terms at normal incidence that fit the table: past it too
+// many cells take the sum in place (2 um: 109 us against 143; 2.6 um, six
+// terms past the table: 141 against 143).
+constexpr double kSerMinTerms = 6.0;
+constexpr size_t kListBlocks = 1280;  // five waves per SIMD, all resident
+// q past which the wavelength sum is used: kSerEps^(1 / 28), 28 terms.
+constexpr float kSerMaxQ = 0.6577f;
+
+struct SeriesArgs {
+    const float4* tab;      // [3 colours][kSerNodes] cubic coefficients of 2 G_c / 81
+    float s0, s1, s2;       // S_c / 81
+    const float4* lines;    // [81] {cmf / 81, 1 / (2 lambda)}
+};
+
+// G_c at the Chebyshev points of every interval: four lanes per interval.
+// The phase is reduced in FP64, the cosine taken in FP32 and summed in FP64.
+__global__ __launch_bounds__(256) void series_table_kernel(const float* __restrict__ cmf,
+                                                           const double* __restrict__ inv_lambda,
+                                                           float* __restrict__ tab) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = t >> 2, j = t & 3;
+    if (i >= kSerNodes) return;             // whole blocks
+    // cos(k pi / 8), k = 0 .. 4; T_n at point m is cos(n (2 m + 1) pi / 8)
+    constexpr double C[5] = {1.0, 0.92387953251128675613, 0.70710678118654752440, 0.38268343236508977173, 0.0};
+    auto cos8 = [&](int k) {                // cos(k pi / 8), any k >= 0
+        k &= 15;
+        if (k > 8) k = 16 - k;
+        return k <= 4 ? C[k] : -C[8 - k];
+    };
+    const double y = (i + 0.5 + 0.5 * cos8(2 * j + 1)) * static_cast<double>(kSerStep);
+    double g[3] = {0.0, 0.0, 0.0};
+#pragma unroll 3
+    for (int k = 0; k < kSpecLambdas; ++k) {
+        double x = y * inv_lambda[k];
+        x -= rint(x);
+        const double c = static_cast<double>(cospif(2.f * static_cast<float>(x)));
+        for (int ch = 0; ch < 3; ++ch) g[ch] += static_cast<double>(cmf[3 * k + ch]) * c;
+    }
+    for (int ch = 0; ch < 3; ++ch) {
+        // the four points' values in every lane of the interval
+        double f[4];
+        for (int m = 0; m < 4; ++m) f[m] = __shfl(g[ch], (threadIdx.x & 60) + m, 64);
+        if (j != 0) continue;
+        // Chebyshev coefficients, then powers of the interval's own variable in [0, 1)
+        double a[4];
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            a[n] = 0.0;
+#pragma unroll
+            for (int m = 0; m < 4; ++m) a[n] += f[m] * cos8(n * (2 * m + 1));
+            a[n] *= n == 0 ? 0.25 : 0.5;
+        }
+        const double b0 = a[0] - a[2], b1 = a[1] - 3.0 * a[3], b2 = 2.0 * a[2], b3 = 4.0 * a[3];
+        const double sc = 2.0 / kSpecLambdas;
+        float* o = tab + (static_cast<size_t>(ch) * kSerNodes + i) * 4;
+        o[0] = static_cast<float>(sc * (b0 - b1 + b2 - b3));
+        o[1] = static_cast<float>(sc * (2.0 * b1 - 4.0 * b2 + 6.0 * b3));
+        o[2] = static_cast<float>(sc * (4.0 * b2 - 12.0 * b3));
+        o[3] = static_cast<float>(sc * 8.0 * b3);
+    }
+}
+
+// The RGB of one cell per lane by the wavelength sum in the square form;
+// the lines come through scalar loads.
+__device__ inline float3 series_direct(const SeriesArgs& sa, float F, float opc) {
+    float x0 = 0.f, x1 = 0.f, x2 = 0.f;
+#pragma unroll 3
+    for (int k = 0; k < kSpecLambdas; ++k) {
+        const float4 l = sa.lines[k];
+        const float c = __builtin_amdgcn_cosf(__builtin_amdgcn_fractf(opc * l.w));
+        const float r = __builtin_amdgcn_rcpf(fmaf(F * c, c, 1.f));
+        x0 = fmaf(r, l.x, x0);
+        x1 = fmaf(r, l.y, x1);
+        x2 = fmaf(r, l.z, x2);
+    }
+    return make_float3(sa.s0 - x0, sa.s1 - x1, sa.s2 - x2);
+}
+
+// One group's inputs, loaded ahead of their use.
+struct SeriesCell {
+    float hi, lo;
+    float2 view;
+};
+
+// The group is wave-uniform: scalar bases, 32-bit lane offsets.  Lanes past
+// the last cell repeat it.
+__device__ inline SeriesCell series_load(const SpecArgs& a, unsigned sg, unsigned lane, unsigned n) {
+    typedef float f2v __attribute__((ext_vector_type(2)));
+    const unsigned base = sg * 64;
+    const unsigned l = min(lane, n - 1 - base);
+    SeriesCell c;
+    c.hi = (a.hi + base)[l];
+    c.lo = (a.lo + base)[l];
+    const f2v v = __builtin_nontemporal_load(reinterpret_cast<const f2v*>(a.view + base) + l);
+    c.view = make_float2(v.x, v.y);
+    return c;
+}
+
+__global__ __launch_bounds__(kSerThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) void spectral_series_kernel(
+    const SpecArgs a, const SeriesArgs sa) {
+    __shared__ float4 tab[3][kSerNodes];
+    __shared__ unsigned s_next;
+    const unsigned lane = threadIdx.x & 63;
+    if (threadIdx.x == 0) s_next = 0;
+    for (int t = threadIdx.x; t < 3 * kSerNodes; t += kSerThreads) (&tab[0][0])[t] = sa.tab[t];
+    const unsigned n = static_cast<unsigned>(a.n);
+    const unsigned last_row = static_cast<unsigned>(a.nt - 1) * static_cast<unsigned>(a.np);
+    const unsigned groups = (n + 63) / 64;
+    const unsigned round_groups = gridDim.x * static_cast<unsigned>(kSerWaves);
+    const unsigned end = (groups + round_groups - 1) / round_groups * round_groups;
+    __syncthreads();
+
+    // The block's groups come in rounds of kSerWaves neighbours, gridDim
+    // blocks to a round, and its waves take them one at a time.  The block's
+    // place in the round moves on from round to round: with a fixed place it
+    // would meet the same columns in every row where a round is a multiple
+    // of the width, and the columns along the silhouette take longer.
+    // Groups past the last one (in the last round) are passed over.
+    auto take = [&]() {
+        unsigned r = 0;
+        if (lane == 0) r = atomicAdd(&s_next, 1u);
+        r = __builtin_amdgcn_readfirstlane(r);
+        const unsigned round = r / static_cast<unsigned>(kSerWaves);
+        const unsigned place = (blockIdx.x + round * kSerSkew) % gridDim.x;
+        return round * round_groups + place * static_cast<unsigned>(kSerWaves) + r % static_cast<unsigned>(kSerWaves);
+    };
+    unsigned sg = take(), next = take();
+    SeriesCell in{0.f, 0.f, make_float2(0.f, 0.f)};
+    if (sg < groups) in = series_load(a, sg, lane, n);
+    while (sg < end) {
+        SeriesCell ahead{0.f, 0.f, make_float2(0.f, 0.f)};
+        if (next < groups) ahead = series_load(a, next, lane, n);
+        const unsigned after = take();
+        if (sg < groups) {
+            const unsigned base = sg * 64;
+            float h = in.hi + in.lo;
+            if (a.pole_virtual && (base < static_cast<unsigned>(a.np) || base + 63 >= last_row)) {
+                const bool top = base + lane < static_cast<unsigned>(a.np);
+                if (top || base + lane >= last_row) {
+                    const float2 m = pole_mean(a.hpole + (top ? 0 : a.ntiles), a.ntiles, static_cast<float>(a.np));
+                    h = m.x + m.y;
+                }
+            }
+            const float q = in.view.x, opc = h * in.view.y;
+            const float u = opc * (1.f / kSerStep);
+            const float K = (1.f - q) * __builtin_amdgcn_rcpf(1.f + q);
+            const bool mine = q <= kSerMaxQ && base + lane < n;      // the others are listed
+            // the terms that matter lie on the table
+            const bool ok = u >= 0.f && __builtin_amdgcn_logf(q) * kSerNodes <= kSerLog2 * u;
+            const float us = mine && ok ? u : 0.f;
+            // Terms in pairs until no lane of the wave needs more; a lane past
+            // its own last term adds terms below its bound (clamped to the
+            // table's last interval).
+            float x0 = 0.f, x1 = 0.f, x2 = 0.f, w = mine && ok ? -q : 0.f, t = us;
+            constexpr float tmax = kSerNodes - 0.5f;
+            auto term = [&]() {
+                const float tc = fminf(t, tmax);
+                const float f = __builtin_amdgcn_fractf(tc);
+                const unsigned i = static_cast<unsigned>(tc);
+                const float4 c0 = tab[0][i], c1 = tab[1][i], c2 = tab[2][i];
+                x0 = fmaf(w, fmaf(fmaf(fmaf(c0.w, f, c0.z), f, c0.y), f, c0.x), x0);
+                x1 = fmaf(w, fmaf(fmaf(fmaf(c1.w, f, c1.z), f, c1.y), f, c1.x), x1);
+                x2 = fmaf(w, fmaf(fmaf(fmaf(c2.w, f, c2.z), f, c2.y), f, c2.x), x2);
+                t += us;
+                w *= -q;
+            };
+            while (__any(fabsf(w) > kSerEps)) {
+                term();
+                term();
+            }
+            if (mine && ok) {
+                // streaming stores, as in spectral_kernel
+                const float e = 1.f - K;
+                float* out = a.rgb + base;
+                __builtin_nontemporal_store(fmaf(sa.s0, e, -K * x0), out + lane);
+                __builtin_nontemporal_store(fmaf(sa.s1, e, -K * x1), out + a.n + lane);
+                __builtin_nontemporal_store(fmaf(sa.s2, e, -K * x2), out + 2 * a.n + lane);
+            }
+            if (__any(mine && !ok)) {
+                const float3 v = series_direct(sa, spec_finesse(q), opc);
+                if (mine && !ok) {
+                    float* out = a.rgb + base;
+                    out[lane] = v.x;
+                    (out + a.n)[lane] = v.y;
+                    (out + 2 * a.n)[lane] = v.z;
+                }
+            }
+        }
+        sg = next;
+        next = after;
+        in = ahead;
+    }
+}
+
+// The view table, and the list of the cells that spectral_series_kernel
+// leaves to spectral_list_kernel (count zeroed before).  1024 cells to a
+// block, one reservation of list entries per block; the order of the blocks'
+// entries does not matter.
+__global__ __launch_bounds__(256) void spectral_view_kernel(const SpecArgs a, float2* __restrict__ out,
+                                                            unsigned* __restrict__ list, unsigned* __restrict__ count) {
+    __shared__ unsigned s_list[1024];
+    __shared__ unsigned s_count, s_at;
+    if (threadIdx.x == 0) s_count = 0;
+    __syncthreads();
+    for (int k = 0; k < 4; ++k) {
+        const size_t cc = blockIdx.x * size_t{1024} + k * 256 + threadIdx.x;
+        if (cc >= a.n) break;
+        int i, j;
+        spec_cell_ij(a, cc, 1.f / static_cast<float>(a.np), i, j);
+        float q, cos_t;
+        spec_view_terms(a, i, j, q, cos_t);
+        out[cc] = make_float2(q, 2e9f * a.n_film * cos_t);
+        if (list && !(q <= kSerMaxQ)) s_list[atomicAdd(&s_count, 1u)] = static_cast<unsigned>(cc);
+    }
+    __syncthreads();
+    if (s_count == 0) return;
+    if (threadIdx.x == 0) s_at = atomicAdd(count, s_count);
+    __syncthreads();
+    for (unsigned t = threadIdx.x; t < s_count; t += 256) list[s_at + t] = s_list[t];
+}
+
+__global__ void zero_count_kernel(unsigned* count) { *count = 0; }
 
 static inline unsigned cdiv_u(size_t a, size_t b) { return static_cast<unsigned>((a + b - 1) / b); }
 
@@ -778,6 +1105,15 @@ constexpr size_t kCmfFrags = 2 * kCmfFragsPerFormat;
 constexpr size_t kCmfPhaseOffset = kCmfFrags * 4 + 4 * kSpecSlots;   // in floats; 8-byte aligned
 constexpr size_t kCmfFloats = kCmfPhaseOffset + 2 * kSpecPhase * 64;
 
+// The series table on the device (floats), behind the fragments: cubics, the
+// lines, 1 / lambda in FP64, the curves.
+constexpr size_t kSerLinesOffset = 12 * static_cast<size_t>(kSerNodes);
+constexpr size_t kSerInvOffset = kSerLinesOffset + 4 * kSpecLambdas;
+constexpr size_t kSerCurvesOffset = kSerInvOffset + 2 * kSpecLambdas;
+constexpr size_t kSerFloats = kSerCurvesOffset + 3 * kSpecLambdas;
+static_assert(4 * kSerNodes % 256 == 0, "table kernel grid");
+static_assert(kCmfFloats % 4 == 0 && kSerInvOffset % 2 == 0, "alignment of the table and of 1 / lambda");
+
 static uint16_t bf16_rne(float x) {
     uint32_t u;
     std::memcpy(&u, &x, 4);
@@ -939,15 +1275,23 @@ static void spectral_prepare(Drainage* d, const float* cmf) {
     if (cmf) {
         for (int k = 0; k < 3 * kSpecLambdas; ++k)
             SF_REQUIRE(std::isfinite(cmf[k]), SF_ERR_INVALID, "colour-matching curve value %d is not finite", k);
-        if (!d->cmf_dev) d->cmf_dev = dalloc_i<float>(kCmfFloats);
+        // Curves equal to the ones in place (by value) are laid out already.
+        if (d->cmf_valid && std::memcmp(cmf, d->cmf_host, sizeof(d->cmf_host)) == 0) return;
+        d->cmf_valid = false;
+        if (!d->cmf_dev) {
+            d->cmf_dev = dalloc_i<float>(kCmfFloats + kSerFloats);
+            d->cmf_series = d->cmf_dev + kCmfFloats;
+        }
         const PackedCmf packed = pack_cmf(cmf);
-        SF_HIP(hipMemcpyAsync(d->cmf_dev, packed.frag.data(), kCmfFrags * sizeof(u32x4), hipMemcpyHostToDevice,
-                              d->stream));
-        SF_HIP(hipMemcpyAsync(d->cmf_dev + kCmfFrags * 4, packed.ulam, sizeof(packed.ulam), hipMemcpyHostToDevice,
-                              d->stream));
-        SF_HIP(hipMemcpyAsync(d->cmf_dev + kCmfPhaseOffset, packed.pfrag, sizeof(packed.pfrag),
-                              hipMemcpyHostToDevice, d->stream));
+        std::vector<float> host(kCmfFloats);
+        std::memcpy(host.data(), packed.frag.data(), kCmfFrags * sizeof(u32x4));
+        std::memcpy(host.data() + kCmfFrags * 4, packed.ulam, sizeof(packed.ulam));
+        std::memcpy(host.data() + kCmfPhaseOffset, packed.pfrag, sizeof(packed.pfrag));
+        SF_HIP(hipMemcpyAsync(d->cmf_dev, host.data(), kCmfFloats * sizeof(float), hipMemcpyHostToDevice, d->stream));
         SF_HIP(hipStreamSynchronize(d->stream));
+        std::memcpy(d->cmf_host, cmf, sizeof(d->cmf_host));
+        d->cmf_valid = true;
+        d->series_valid = false;
         for (int f = 0; f < 2; ++f) {
             for (int c = 0; c < 3; ++c) d->cmf_sum[f][c] = packed.sum[f][c];
             d->cmf_lo[f] = packed.has_lo[f];
@@ -966,6 +1310,34 @@ static int spectral_format(const Drainage* d) {
         return 1;
     }
     return (d->cmf_f16_range && d->cmf_f16_bound) ? 1 : 0;
+}
+
+// The series table of the curves in place, built on the first series pass
+// that uses them.
+static void ensure_series(Drainage* d) {
+    if (d->series_valid) return;
+    float host[kSerFloats - kSerLinesOffset];
+    for (int k = 0; k < kSpecLambdas; ++k) {
+        for (int c = 0; c < 3; ++c)
+            host[4 * k + c] = static_cast<float>(d->cmf_host[3 * k + c] / static_cast<double>(kSpecLambdas));
+        host[4 * k + 3] = static_cast<float>(0.5 / (380.0 + 5.0 * k));
+    }
+    double inv[kSpecLambdas];
+    for (int k = 0; k < kSpecLambdas; ++k) inv[k] = 1.0 / (380.0 + 5.0 * k);
+    std::memcpy(host + (kSerInvOffset - kSerLinesOffset), inv, sizeof(inv));
+    std::memcpy(host + (kSerCurvesOffset - kSerLinesOffset), d->cmf_host, sizeof(d->cmf_host));
+    SF_HIP(hipMemcpyAsync(d->cmf_series + kSerLinesOffset, host, sizeof(host), hipMemcpyHostToDevice, d->stream));
+    for (int c = 0; c < 3; ++c) {
+        double sum = 0.0;
+        for (int k = 0; k < kSpecLambdas; ++k) sum += d->cmf_host[3 * k + c];
+        d->cmf_mean[c] = static_cast<float>(sum / kSpecLambdas);
+    }
+    hipLaunchKernelGGL(series_table_kernel, dim3(4 * kSerNodes / 256), dim3(256), 0, d->stream,
+                       d->cmf_series + kSerCurvesOffset, reinterpret_cast<const double*>(d->cmf_series + kSerInvOffset),
+                       d->cmf_series);
+    SF_HIP(hipGetLastError());
+    SF_HIP(hipStreamSynchronize(d->stream));        // `host` is read until here
+    d->series_valid = true;
 }
 
 // Launches spectral_kernel on stream st over the context's current state
@@ -1007,28 +1379,61 @@ void spectral_launch(Drainage* d, const sf_camera* cam, double n_film, const flo
     a.view = nullptr;
     // View terms of this camera and film index, cached on the context.
     const float key[6] = {a.cx, a.cy, a.cz, a.radius, a.n_film, a.inv_n_film};
-    if (!d->spec_view) d->spec_view = dalloc_i<float2>(d->n);
+    const bool large = d->n >= kSerMinCells && d->n < (size_t{1} << 31);      // 32-bit cell indices
+    if (!d->spec_view) {
+        // the view table, and behind it the list of near-grazing cells and its length
+        d->spec_view = dalloc_i<float2>(d->n + (large ? d->n / 2 + 1 : 0));
+        if (large) d->spec_list = reinterpret_cast<unsigned*>(d->spec_view + d->n);
+    }
     if (!d->spec_view_valid || std::memcmp(key, d->spec_view_key, sizeof(key)) != 0) {
-        hipLaunchKernelGGL(spectral_view_kernel, dim3(cdiv_u(d->n, 256)), dim3(256), 0, st, a, d->spec_view);
+        unsigned* count = d->spec_list ? d->spec_list + d->n : nullptr;
+        if (count) hipLaunchKernelGGL(zero_count_kernel, dim3(1), dim3(1), 0, st, count);
+        hipLaunchKernelGGL(spectral_view_kernel, dim3(cdiv_u(d->n, 1024)), dim3(256), 0, st, a, d->spec_view,
+                           d->spec_list, count);
         SF_HIP(hipGetLastError());
         std::memcpy(d->spec_view_key, key, sizeof(key));
         d->spec_view_valid = true;
     }
     a.view = d->spec_view;
-    const size_t supergroups = (d->n + 63) / 64;
-    // About two 64-cell groups per wave: the short blocks balance the tail
-    // (145.8 us at 2048 x 4096, against 154.5 us with 2560 grid-striding
-    // blocks and 149.5 us with one group per wave).
-    const unsigned blocks = static_cast<unsigned>(std::max<size_t>(1, (supergroups + 7) / 8));
-    static void (*const kernels[2][kSpecMaxSkip + 1])(const SpecArgs) = {
-        {spectral_kernel<false, 0>, spectral_kernel<false, 1>, spectral_kernel<false, 2>},
-        {spectral_kernel<true, 0>, spectral_kernel<true, 1>, spectral_kernel<true, 2>}};
-    void (*kern)(const SpecArgs) = kernels[f][d->cmf_skip];
-    if (d->spec_timer.enabled) {
-        auto& ev = d->spec_timer.next(st);
-        hipExtLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, st, ev.first, ev.second, 0, a);
+    const size_t groups = (d->n + 63) / 64;
+    if (d->spec_operand == SF_SPECTRAL_OPERAND_AUTO && large &&
+        d->h_max * 2e9 * n_film * kSerMinTerms <= kSerNodes * static_cast<double>(kSerStep)) {
+        ensure_series(d);
+        // As many blocks as are resident (two per CU by their waves), each
+        // wave walking several groups on the block's copy of the table.
+        const size_t want = (groups + kSerWaves - 1) / kSerWaves;
+        const dim3 grid(static_cast<unsigned>(std::min<size_t>(want, kSerBlocks)));
+        const SeriesArgs sa{reinterpret_cast<const float4*>(d->cmf_series), d->cmf_mean[0], d->cmf_mean[1],
+                            d->cmf_mean[2], reinterpret_cast<const float4*>(d->cmf_series + kSerLinesOffset)};
+        static void (*const kernels[2][kSpecMaxSkip + 1])(const SpecArgs, const unsigned*, const unsigned*) = {
+            {spectral_list_kernel<false, 0>, spectral_list_kernel<false, 1>, spectral_list_kernel<false, 2>},
+            {spectral_list_kernel<true, 0>, spectral_list_kernel<true, 1>, spectral_list_kernel<true, 2>}};
+        void (*rest)(const SpecArgs, const unsigned*, const unsigned*) = kernels[f][d->cmf_skip];
+        const dim3 rest_grid(static_cast<unsigned>(std::min<size_t>((groups + 3) / 4, kListBlocks)));
+        const unsigned* count = d->spec_list + d->n;
+        if (d->spec_timer.enabled) {      // one interval over both launches
+            auto& ev = d->spec_timer.next(st);
+            hipExtLaunchKernelGGL(spectral_series_kernel, grid, dim3(kSerThreads), 0, st, ev.first, nullptr, 0, a, sa);
+            hipExtLaunchKernelGGL(rest, rest_grid, dim3(256), 0, st, nullptr, ev.second, 0, a, d->spec_list, count);
+        } else {
+            hipLaunchKernelGGL(spectral_series_kernel, grid, dim3(kSerThreads), 0, st, a, sa);
+            hipLaunchKernelGGL(rest, rest_grid, dim3(256), 0, st, a, d->spec_list, count);
+        }
     } else {
-        hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, st, a);
+        // About two 64-cell groups per wave: the short blocks balance the tail
+        // (145.8 us at 2048 x 4096, against 154.5 us with 2560 grid-striding
+        // blocks and 149.5 us with one group per wave).
+        static void (*const kernels[2][kSpecMaxSkip + 1])(const SpecArgs) = {
+            {spectral_kernel<false, 0>, spectral_kernel<false, 1>, spectral_kernel<false, 2>},
+            {spectral_kernel<true, 0>, spectral_kernel<true, 1>, spectral_kernel<true, 2>}};
+        void (*kern)(const SpecArgs) = kernels[f][d->cmf_skip];
+        const dim3 grid(static_cast<unsigned>(std::max<size_t>(1, (groups + 7) / 8)));
+        if (d->spec_timer.enabled) {
+            auto& ev = d->spec_timer.next(st);
+            hipExtLaunchKernelGGL(kern, grid, dim3(256), 0, st, ev.first, ev.second, 0, a);
+        } else {
+            hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, a);
+        }
     }
     SF_HIP(hipGetLastError());
 }

@@ -384,3 +384,76 @@ def test_step_spectral_matches_serial(oracle, nt, npf, steps, flags):
     err = np.max(np.abs(rgb_a.reshape(3, -1)[:, cells].T - want))
     print("step_spectral %dx%d after %d steps: max |rgb - oracle| = %.3g" % (nt, npf, steps, err))
     assert err <= 1e-3
+
+
+def _series_bound(cm, q_max=0.66):
+    """Largest error of the cosine-series spectral pass per channel: the
+    terms left out (1.6e-5 of the mean |cmf|), the cubic table's (2 pi 32 /
+    lambda)^4 / 3072 of each wavelength's share times 2 q / (1 + q), the FP16
+    rounding of the cells that keep the wavelength sum (2^-18 sum |cmf|,
+    1e-5 of skipped slots), and 2e-5 for the FP32 optical path."""
+    a = np.abs(cm.astype(np.float64))
+    lam = 380.0 + 5.0 * np.arange(81)
+    table = (a * ((2.0 * np.pi * 32.0 / lam) ** 4 / 3072.0)[:, None]).sum(axis=0) / 81.0 * 2.0 * q_max / (1.0 + q_max)
+    series = 1.6e-5 * a.sum(axis=0) / 81.0 + table
+    return np.maximum(series, 2.0 ** -18 * a.sum(axis=0) + 1e-5) + 2e-5
+
+
+@pytest.mark.parametrize("nt,npf,film,lines", [
+    (1024, 1024, "normal", False),     # the smallest grid of the series
+    (1027, 1031, "normal", False),     # rows and groups of 64 do not meet, a partial last group
+    (1027, 1031, "thin", False),       # 0-50 nm, with cells of no thickness
+    (1031, 1100, "thick", False),      # up to 1.9 um: some cells past the table
+    (1024, 1024, "micron60", False),   # past the series: the wavelength sum
+    (1024, 1024, "normal", True),      # one wavelength per curve: no decay of the sums with the path
+    (600, 4096, "normal", False),
+])
+def test_spectral_series(oracle, nt, npf, film, lines):
+    ctx, h0, p, cam, cmf = _spectral_case(nt, npf, 21)
+    h = {"normal": h0, "thin": h0 * 0.05, "thick": h0 * (1.9e-6 / h0.max()), "micron60": h0 * 60.0}[film].copy()
+    rng = np.random.default_rng(4)
+    if film == "thin":
+        h.reshape(-1)[rng.choice(h.size, 500, replace=False)] = 0.0
+    ctx.set_fields(h, np.full_like(h, 0.5))
+    h = ctx.fields()[0]
+    cm = cmf.astype(np.float32)
+    if lines:
+        cm = np.zeros_like(cm)
+        cm[10, 0] = cm[41, 1] = cm[70, 2] = 1.0
+    got = spectral_rgb(ctx, cam, cm)
+    cells = np.unique(np.concatenate([rng.choice(nt * npf, 20000, replace=False), np.arange(npf),
+                                      nt * npf - 1 - np.arange(npf)]))
+    want = oracle.spectral_cells(h, cells, p.bubble_radius, cam, 1.33, cm.astype(np.float64))
+    err = np.max(np.abs(got.reshape(3, -1)[:, cells].T - want), axis=0)
+    # a 60 um film's path, 160 um in FP32, is off by 1e-5 um: 1.5e-4 of phase and times the slope of the sum
+    bound = _series_bound(cm) + (1e-3 if film == "micron60" else 0.0)
+    print("series %dx%d %s: max err %s (bound %s)" % (nt, npf, film, err, bound))
+    assert np.all(err <= bound)
+
+
+def test_spectral_series_state_and_curves(oracle):
+    """The series on a stepped state (lazy pole rows), and with curves and
+    cameras exchanged between calls."""
+    nt, npf = 1024, 2048
+    ctx, h0, p, cam, cmf = _spectral_case(nt, npf, 23)
+    cm = cmf.astype(np.float32)
+    other = (cm * np.float32(0.5))[:, ::-1].copy()
+    camera = L.Camera()
+    for k in range(3):
+        camera.position[k] = cam[k]
+    L.check(L.lib().sf_drainage_step_spectral(ctx.handle, 3, 0.0, C.byref(camera), 1.33, L.fptr(cm)))
+    got = np.empty((3, nt, npf), np.float32)
+    L.check(L.lib().sf_spectral_copy_rgb(ctx.handle, L.fptr(got)))
+    h = ctx.fields()[0]
+    cells = np.concatenate([np.arange(2 * npf), (nt - 2) * npf + np.arange(2 * npf),
+                            np.random.default_rng(1).choice(nt * npf, 5000, replace=False)])
+    cam2 = (-cam[1], cam[2], cam[0])
+    for c, m in ((cam, cm), (cam2, cm), (cam2, other), (cam, other), (cam, cm)):
+        if m is not cm or c is not cam:
+            got = spectral_rgb(ctx, c, m)
+        want = oracle.spectral_cells(h, cells, p.bubble_radius, c, 1.33, m.astype(np.float64))
+        err = np.max(np.abs(got.reshape(3, -1)[:, cells].T - want), axis=0)
+        assert np.all(err <= _series_bound(m)), (c, err)
+        got = spectral_rgb(ctx, cam, cm)
+    again = spectral_rgb(ctx, cam, cm)
+    assert np.array_equal(got, again)
