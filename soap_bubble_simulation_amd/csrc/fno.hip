@@ -46,6 +46,8 @@ namespace {
 constexpr double kPi = 3.14159265358979323846;
 constexpr int kCin = kLiftIn;
 constexpr int kCout = kProjOut;
+constexpr int kBackBlocks = 512;          // blocks of the fused backward kernel (two per CU, each walks rows)
+constexpr long long kLiftFewRows = 8192;
 constexpr int kSplitRows = 4096;          // rows per split-K chunk of the weight gradients
 
 template <class T>
@@ -387,6 +389,8 @@ struct Fno {
     float* Iphi = nullptr;     // [P][2 Mp]
     unsigned short* Ephi16 = nullptr;   // Ephi and Iphi rounded to BF16 (the
     unsigned short* Iphi16 = nullptr;   // fused layer kernel's MFMA operands)
+    unsigned short* EphiT16 = nullptr;  // their transposes (the fused backward kernel's)
+    unsigned short* IphiT16 = nullptr;
     unsigned short* Eth16 = nullptr;    // Eth and Ath rounded to BF16 (the fused
     unsigned short* Ath16 = nullptr;    // inference theta stage's MFMA operands)
     float* wfold = nullptr;             // layer-0 weights with the lift folded in ([C][C] + [C])
@@ -428,7 +432,7 @@ struct Fno {
 
     ~Fno() {
         if (stream) (void)hipStreamSynchronize(stream);
-        void* ps[] = {w, grad, adam_m, adam_v, Ephi, Esum, Eth, Ath, Iphi, Ephi16, Iphi16, Eth16, Ath16, wfold, in, out, target, dout, ybuf, X1, G, Y, Z,
+        void* ps[] = {w, grad, adam_m, adam_v, Ephi, Esum, Eth, Ath, Iphi, Ephi16, Iphi16, EphiT16, IphiT16, Eth16, Ath16, wfold, in, out, target, dout, ybuf, X1, G, Y, Z,
                       dxa, dxb, dz, dXs, part, loss_part, dscratch, ht_hi, ht_lo, ha_hi, ha_lo, hb_hi, hb_lo,
                       sel_hi, sel_lo, hp_hi, hp_lo, d_win, feat_rows, d_take, rpart};
         for (void* p : ps) (void)hipFree(p);
@@ -548,6 +552,17 @@ struct Fno {
         Iphi16 = galloc<unsigned short>(i16.size());
         SF_HIP(hipMemcpy(Ephi16, e16.data(), e16.size() * 2, hipMemcpyHostToDevice));
         SF_HIP(hipMemcpy(Iphi16, i16.data(), i16.size() * 2, hipMemcpyHostToDevice));
+        auto transposed = [](const std::vector<unsigned short>& v, int r, int c) {      // v [r][c]
+            std::vector<unsigned short> o(v.size());
+            for (int i = 0; i < r; ++i)
+                for (int j = 0; j < c; ++j) o[static_cast<size_t>(j) * r + i] = v[static_cast<size_t>(i) * c + j];
+            return o;
+        };
+        const std::vector<unsigned short> eT = transposed(e16, 2 * Mp, P), iT = transposed(i16, P, 2 * Mp);
+        EphiT16 = galloc<unsigned short>(eT.size());
+        IphiT16 = galloc<unsigned short>(iT.size());
+        SF_HIP(hipMemcpy(EphiT16, eT.data(), eT.size() * 2, hipMemcpyHostToDevice));
+        SF_HIP(hipMemcpy(IphiT16, iT.data(), iT.size() * 2, hipMemcpyHostToDevice));
         const std::vector<unsigned short> et16 = bf16(eth), at16 = bf16(ath);
         Eth16 = galloc<unsigned short>(et16.size());
         Ath16 = galloc<unsigned short>(at16.size());
@@ -643,17 +658,38 @@ struct Fno {
     using RowKernel = void (*)(RowArgs);
 
     // Fused layer kernel for this shape, or null (then the unfused GEMM path
-    // runs): n_phi 512 (8 waves x 4 row tiles) or 128 (4 waves x 2), width
-    // 16 or 32, 2 modes_phi 16 or 32.  row_threads receives the block size.
+    // runs): n_phi 512 (8 waves x 4 row tiles), 256 (4 x 4) or 128 (4 x 2),
+    // width 16 or 32, 2 modes_phi 16 or 32.  row_threads receives the block size.
     RowKernel row_kernel(int* row_threads) const {
         const int CT = C / 16, JT = (2 * Mp) / 16;
         if (C % 16 || (2 * Mp) % 16) return nullptr;
 #define SF_ROWK(p, r, w, c, j) \
     if (P == p && CT == c && JT == j) { *row_threads = 64 * w; return &fno_row_kernel<r, c, j, w>; }
         SF_ROWK(512, 4, 8, 2, 2) SF_ROWK(512, 4, 8, 1, 1) SF_ROWK(512, 4, 8, 2, 1) SF_ROWK(512, 4, 8, 1, 2)
+        SF_ROWK(256, 4, 4, 2, 2) SF_ROWK(256, 4, 4, 1, 1) SF_ROWK(256, 4, 4, 2, 1) SF_ROWK(256, 4, 4, 1, 2)
         SF_ROWK(128, 2, 4, 2, 2) SF_ROWK(128, 2, 4, 1, 1) SF_ROWK(128, 2, 4, 2, 1) SF_ROWK(128, 2, 4, 1, 2)
 #undef SF_ROWK
         return nullptr;
+    }
+
+    using RowBackKernel = void (*)(RowBackArgs);
+
+    // Fused backward kernels (top, mid, bottom) of the shapes of row_kernel.
+    bool row_back_kernels(RowBackKernel (&k)[3]) const {
+        const int CT = C / 16, JT = (2 * Mp) / 16;
+        if (C % 16 || (2 * Mp) % 16) return false;
+#define SF_BACKK(p, r, w, c, j)                                                                        \
+    if (P == p && CT == c && JT == j) {                                                               \
+        k[0] = &fno_row_back_kernel<r, c, j, w, kBackTop>;                                            \
+        k[1] = &fno_row_back_kernel<r, c, j, w, kBackMid>;                                            \
+        k[2] = &fno_row_back_kernel<r, c, j, w, kBackBottom>;                                         \
+        return true;                                                                                  \
+    }
+        SF_BACKK(512, 4, 8, 2, 2) SF_BACKK(512, 4, 8, 1, 1) SF_BACKK(512, 4, 8, 2, 1) SF_BACKK(512, 4, 8, 1, 2)
+        SF_BACKK(256, 4, 4, 2, 2) SF_BACKK(256, 4, 4, 1, 1) SF_BACKK(256, 4, 4, 2, 1) SF_BACKK(256, 4, 4, 1, 2)
+        SF_BACKK(128, 2, 4, 2, 2) SF_BACKK(128, 2, 4, 1, 1) SF_BACKK(128, 2, 4, 2, 1) SF_BACKK(128, 2, 4, 1, 2)
+#undef SF_BACKK
+        return false;
     }
 
     // theta stage of layer l: X1 (phi DFT of x_l) -> Z (inverse theta DFT of
@@ -733,6 +769,26 @@ struct Fno {
         SF_HIP(hipGetLastError());
     }
 
+    // Layer-0 phi DFT of the lifted features (X1) for B bubbles.
+    void lift_dft(int B) {
+        const int J = 2 * Mp;
+        const size_t lds = static_cast<size_t>(P * kCin + J * (kCin + 1)) * sizeof(float);
+        SF_REQUIRE(lds <= 64 * 1024 && P <= kLiftDftMaxP, SF_ERR_INTERNAL, "lift DFT tile too large");
+        const long long nrows = static_cast<long long>(B) * T;
+        if (P % 16 == 0 && J == kLiftWaveJ && 64 % C == 0) {
+            // Four rows per wave share each load of the table; two where four
+            // would leave most of the chip's 1024 SIMDs with one wave or none.
+            const bool few = nrows <= kLiftFewRows;
+            const int per = 4 * (few ? 2 : 4);
+            hipLaunchKernelGGL((few ? lift_dft_wave_kernel<kCin, 2> : lift_dft_wave_kernel<kCin, 4>),
+                               dim3(static_cast<unsigned>((nrows + per - 1) / per)), dim3(256), 0, stream, in, Ephi,
+                               Esum, w + o_wl, w + o_bl, X1, P, C, nrows);
+        } else
+            hipLaunchKernelGGL(lift_dft_kernel<kCin>, dim3(static_cast<unsigned>(B * T)), dim3(256), lds, stream, in,
+                               Ephi, w + o_wl, w + o_bl, X1, P, J, C);
+        SF_HIP(hipGetLastError());
+    }
+
     // training: keep the pre-activations for the backward pass
     void forward(int B, bool training) {
         const long long R = static_cast<long long>(B) * N;
@@ -742,18 +798,8 @@ struct Fno {
             // Inference: the lift is folded into the layer-0 phi DFT and the
             // layer-0 row kernel, and the projection into the last one, so
             // neither x_0 nor x_L is written or read.
-            const int J = 2 * Mp;
-            const size_t lds = static_cast<size_t>(P * kCin + J * (kCin + 1)) * sizeof(float);
-            SF_REQUIRE(lds <= 64 * 1024 && P <= kLiftDftMaxP, SF_ERR_INTERNAL, "lift DFT tile too large");
+            lift_dft(B);
             const long long nrows = static_cast<long long>(B) * T;
-            if (P % 16 == 0 && J == kLiftWaveJ && 64 % C == 0)
-                hipLaunchKernelGGL(lift_dft_wave_kernel<kCin>,
-                                   dim3(static_cast<unsigned>((nrows + 4 * kLiftRows - 1) / (4 * kLiftRows))), dim3(256),
-                                   0, stream, in, Ephi, Esum, w + o_wl, w + o_bl, X1, P, C, nrows);
-            else
-                hipLaunchKernelGGL(lift_dft_kernel<kCin>, dim3(static_cast<unsigned>(B * T)), dim3(256), lds, stream, in,
-                                   Ephi, w + o_wl, w + o_bl, X1, P, J, C);
-            SF_HIP(hipGetLastError());
             for (int l = 0; l < L; ++l) {
                 const RowWaveKernel wk = row_wave_kernel(l, L);
                 theta_stage_inference(l, B);
@@ -779,28 +825,31 @@ struct Fno {
             }
             return;
         }
+        if (rk) {
+            // The lift is folded into the first phi DFT and the first row
+            // kernel, the projection into the last; every layer keeps its
+            // pre-activations and its output (FP32) for the backward pass.
+            lift_dft(B);
+            for (int l = 0; l < L; ++l) {
+                theta_stage(l, B);
+                const bool last = l == L - 1;
+                RowArgs ra{xs[l], Z, w + o_w[l], w + o_b[l], Iphi16, Ephi16, xs[l + 1], zs[l], last ? nullptr : X1,
+                           last ? 0 : 1, l == 0 ? in : nullptr, w + o_wl, w + o_bl, w + o_q, w + o_qb,
+                           last ? out : nullptr, 0};
+                hipLaunchKernelGGL(rk, dim3(static_cast<unsigned>(B * T)), dim3(row_threads), 0, stream, ra);
+                SF_HIP(hipGetLastError());
+            }
+            return;
+        }
         // lift (FP32, bias included)
         hipLaunchKernelGGL(lift_kernel<kCin>, dim3(blocks_for(R * ((C + 3) / 4), 256, 16384)), dim3(256), 0, stream, in,
                            w + o_wl, w + o_bl, xs[0], R, C);
         SF_HIP(hipGetLastError());
-        if (rk) {
-            const int MpC2 = 2 * Mp * C;
-            gemm(Ephi, xs[0], X1, 2 * Mp, C, P, P, C, C, 0, static_cast<long long>(P) * C,
-                 static_cast<long long>(MpC2), B * T, 0, 0, 1.f, 0.f);
-            for (int l = 0; l < L; ++l) {
-                theta_stage(l, B);
-                RowArgs ra{xs[l], Z, w + o_w[l], w + o_b[l], Iphi16, Ephi16, xs[l + 1], training ? zs[l] : nullptr,
-                           l < L - 1 ? X1 : nullptr, l < L - 1 ? 1 : 0};
-                hipLaunchKernelGGL(rk, dim3(static_cast<unsigned>(B * T)), dim3(row_threads), 0, stream, ra);
-                SF_HIP(hipGetLastError());
-            }
-        } else {
-            for (int l = 0; l < L; ++l) {
-                spectral_forward(l, B, xs[l]);
-                gemm(xs[l], w + o_w[l], zs[l], static_cast<int>(R), C, C, C, C, C, 0, 0, 0, 1, 0, 0, 1.f, 0.f);
-                hipLaunchKernelGGL(bias_act_kernel, dim3(blocks_for(R * C, 256, 16384)), dim3(256), 0, stream, zs[l],
-                                   ybuf, w + o_b[l], xs[l + 1], R * C, C, l < L - 1 ? 1 : 0);
-            }
+        for (int l = 0; l < L; ++l) {
+            spectral_forward(l, B, xs[l]);
+            gemm(xs[l], w + o_w[l], zs[l], static_cast<int>(R), C, C, C, C, C, 0, 0, 0, 1, 0, 0, 1.f, 0.f);
+            hipLaunchKernelGGL(bias_act_kernel, dim3(blocks_for(R * C, 256, 16384)), dim3(256), 0, stream, zs[l],
+                               ybuf, w + o_b[l], xs[l + 1], R * C, C, l < L - 1 ? 1 : 0);
         }
         // projection (FP32, bias included)
         hipLaunchKernelGGL(project_kernel<kCout>, dim3(blocks_for(R, 256, 16384)), dim3(256), 0, stream, xs[L],
@@ -822,11 +871,82 @@ struct Fno {
         return s / static_cast<double>(n);
     }
 
+    // Adjoint of theta_stage: Z (gradient at the inverse phi DFT's input) ->
+    // X1 (gradient at the phi coefficients); accumulates the gradient of R.
+    void theta_backward(int l, int B) {
+        const int MpC2 = 2 * Mp * C;
+        gemm(Ath, Z, Y, 2 * Mt, Mp * C, 2 * T, 2 * Mt, Mp * C, Mp * C, 0, static_cast<long long>(2 * T) * Mp * C,
+             static_cast<long long>(2 * Mt) * Mp * C, B, 1, 0, 1.f, 0.f);
+        hipLaunchKernelGGL(mode_mix_grad_kernel, dim3(Mt * Mp), dim3(256), 0, stream, spec[l], w + o_r[l], Y, dXs,
+                           grad + o_r[l], B, Mt, Mp, C);
+        const long long tot = static_cast<long long>(B) * Mt * Mp * C;
+        hipLaunchKernelGGL(theta_combine_adjoint_kernel, dim3(blocks_for(tot)), dim3(256), 0, stream, dXs, G, Mt,
+                           Mp, C, tot);
+        gemm(Eth, G, X1, T, MpC2, 2 * Mt, T, MpC2, MpC2, 0, static_cast<long long>(2 * Mt) * MpC2,
+             static_cast<long long>(T) * MpC2, B, 1, 0, 1.f, 0.f);
+        SF_HIP(hipGetLastError());
+    }
+
+    // Backward pass of the shapes with a fused row kernel: a launch per layer
+    // (fno_row_back_kernel) and the adjoint theta stage between them.
+    void backward_fused(int B, RowBackKernel (&bk)[3], int threads) {
+        const int nrows = B * T;
+        const int nblk = std::min(nrows, kBackBlocks);
+        const int cols = C * C + C, cols_q = C * kCout + kCout;
+        const long long need = static_cast<long long>(nblk) * (cols + cols_q);
+        if (need > part_cap) {
+            (void)hipFree(part);
+            part = nullptr;
+            part_cap = 0;
+            part = galloc<float>(need);
+            part_cap = need;
+        }
+        float* part_q = part + static_cast<long long>(nblk) * cols;
+        auto fold = [&](const float* src, int n, float* dst) {
+            hipLaunchKernelGGL(column_sum_kernel, dim3((n + 31) / 32), dim3(256), 0, stream, src,
+                               static_cast<long long>(nblk), n, dst, 1);
+            SF_HIP(hipGetLastError());
+        };
+        for (int l = L; l >= 0; --l) {        // launch l ends at layer l - 1's pre-activations
+            if (l < L) theta_backward(l, B);
+            RowBackArgs a{};
+            a.dz = dz;
+            a.X1 = X1;
+            a.W = l < L ? w + o_w[l] : nullptr;
+            a.EphiT = EphiT16;
+            a.IphiT = IphiT16;
+            a.z = l > 0 && l < L ? zs[l - 1] : nullptr;
+            a.x = l > 1 ? xs[l - 1] : nullptr;
+            a.in = in;
+            a.Wl = w + o_wl;
+            a.bl = w + o_bl;
+            a.xL = xs[L];
+            a.dout = dout;
+            a.Q = w + o_q;
+            a.dz_out = dz;
+            a.Z_out = Z;
+            a.part = part;
+            a.part_q = part_q;
+            a.rows = nrows;
+            hipLaunchKernelGGL(bk[l == L ? kBackTop : (l > 0 ? kBackMid : kBackBottom)], dim3(nblk), dim3(threads), 0,
+                               stream, a);
+            SF_HIP(hipGetLastError());
+            if (l == L) fold(part_q, cols_q, grad + o_q);
+            fold(part, l > 0 ? cols : kCin * C + C, grad + (l > 0 ? o_w[l - 1] : o_wl));
+        }
+    }
+
     void backward(int B) {
         const long long R = static_cast<long long>(B) * N;
         const int MpC2 = 2 * Mp * C;
         hipLaunchKernelGGL(fill_f32_kernel, dim3(blocks_for(n_params, 256, 16384)), dim3(256), 0, stream, grad,
                            n_params, 0.f);
+        RowBackKernel bk[3];
+        int row_threads = 0;
+        if (row_kernel(&row_threads) && row_back_kernels(bk)) {
+            backward_fused(B, bk, row_threads);
+            return;
+        }
         // projection
         weight_grad(xs[L], dout, R, C, kCout, grad + o_q);
         bias_grad(dout, R, kCout, grad + o_qb);
@@ -839,18 +959,9 @@ struct Fno {
             bias_grad(dz, R, C, grad + o_b[l]);
             weight_grad(xs[l], dz, R, C, C, grad + o_w[l]);
             gemm(dz, w + o_w[l], dxn, static_cast<int>(R), C, C, C, C, C, 0, 0, 0, 1, 0, 1, 1.f, 0.f);
-            // adjoint of the spectral path
             gemm(Iphi, dz, Z, 2 * Mp, C, P, 2 * Mp, C, C, 0, static_cast<long long>(P) * C,
                  static_cast<long long>(MpC2), B * T, 1, 0, 1.f, 0.f);
-            gemm(Ath, Z, Y, 2 * Mt, Mp * C, 2 * T, 2 * Mt, Mp * C, Mp * C, 0, static_cast<long long>(2 * T) * Mp * C,
-                 static_cast<long long>(2 * Mt) * Mp * C, B, 1, 0, 1.f, 0.f);
-            hipLaunchKernelGGL(mode_mix_grad_kernel, dim3(Mt * Mp), dim3(256), 0, stream, spec[l], w + o_r[l], Y, dXs,
-                               grad + o_r[l], B, Mt, Mp, C);
-            const long long tot = static_cast<long long>(B) * Mt * Mp * C;
-            hipLaunchKernelGGL(theta_combine_adjoint_kernel, dim3(blocks_for(tot)), dim3(256), 0, stream, dXs, G, Mt,
-                               Mp, C, tot);
-            gemm(Eth, G, X1, T, MpC2, 2 * Mt, T, MpC2, MpC2, 0, static_cast<long long>(2 * Mt) * MpC2,
-                 static_cast<long long>(T) * MpC2, B, 1, 0, 1.f, 0.f);
+            theta_backward(l, B);
             gemm(Ephi, X1, dxn, P, C, 2 * Mp, P, C, C, 0, static_cast<long long>(MpC2), static_cast<long long>(P) * C,
                  B * T, 1, 0, 1.f, 1.f);
             std::swap(dx, dxn);

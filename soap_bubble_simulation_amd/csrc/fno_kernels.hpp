@@ -138,6 +138,24 @@ __device__ inline float gelu(float z) {      // tanh form
     return 0.5f * z * (1.f + tanhf(k0 * (z + k1 * z * z * z)));
 }
 
+__device__ inline float gelu_exp(float z) {
+    // 0.5 z (1 + tanh u) = z / (1 + exp(-2u)), u = k0 (z + k1 z^3); hardware
+    // exp2 and reciprocal (about 1e-6 relative, far below the BF16 rounding
+    // the result is stored with)
+    const float k0 = 0.7978845608028654f, k1 = 0.044715f;
+    const float u = k0 * fmaf(k1 * z, z * z, z);
+    const float e = __builtin_amdgcn_exp2f(-2.8853900817779268f * u);
+    return z * __builtin_amdgcn_rcpf(1.f + e);
+}
+
+// Derivative of gelu_exp with s = 1 / (1 + exp(-2u)) = (1 + tanh u) / 2.
+__device__ inline float gelu_exp_grad(float z) {
+    const float k0 = 0.7978845608028654f, k1 = 0.044715f;
+    const float u = k0 * fmaf(k1 * z, z * z, z);
+    const float s = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-2.8853900817779268f * u));
+    return fmaf(2.f * k0 * z * fmaf(3.f * k1 * z, z, 1.f), s * (1.f - s), s);
+}
+
 // ---- fused Fourier layer, one block per (bubble, theta row) ------------------
 //
 // For one grid row t of bubble b (P cells x C channels):
@@ -265,7 +283,7 @@ __global__ __launch_bounds__(64 * WAVES) void fno_row_kernel(const RowArgs a) {
             for (int v = 0; v < 4; ++v) {
                 const int p = wave * RT * 16 + rt * 16 + kq + v;
                 const float z = acc[rt][ct][v] + bo;
-                const float xv = a.act ? gelu(z) : z;
+                const float xv = a.act ? gelu_exp(z) : z;
                 if (xo) xo[static_cast<long long>(p) * C + o] = xv;
                 if (xo16) xo16[static_cast<long long>(p) * C + o] = to_bf16(xv);
                 if (zo) zo[static_cast<long long>(p) * C + o] = z;
@@ -385,16 +403,6 @@ __global__ __launch_bounds__(256) void lift_fold_kernel(const float* __restrict_
             bf[n] = v;
         }
     }
-}
-
-__device__ inline float gelu_exp(float z) {
-    // 0.5 z (1 + tanh u) = z / (1 + exp(-2u)), u = k0 (z + k1 z^3); hardware
-    // exp2 and reciprocal (about 1e-6 relative, far below the BF16 rounding
-    // the result is stored with)
-    const float k0 = 0.7978845608028654f, k1 = 0.044715f;
-    const float u = k0 * fmaf(k1 * z, z * z, z);
-    const float e = __builtin_amdgcn_exp2f(-2.8853900817779268f * u);
-    return z * __builtin_amdgcn_rcpf(1.f + e);
 }
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -703,30 +711,29 @@ __global__ __launch_bounds__(256) void lift_dft_kernel(const float* __restrict__
 }
 
 // The same product on FP32 MFMA (v_mfma_f32_16x16x4_f32, lane l supplies
-// A[l % 16][l / 16] and B[l / 16][l % 16]), one wave per kLiftRows rows of a
-// bubble's grid, so each 16-byte load of the Ephi rows (A) serves kLiftRows
+// A[l % 16][l / 16] and B[l / 16][l % 16]), one wave per ROWS rows of a
+// bubble's grid, so each 16-byte load of the Ephi rows (A) serves ROWS
 // products: S_r = Ephi in_r (J x NIN, K = P split so that lane group g sums
 // cells g P/4 .. (g + 1) P/4 - 1), two rows per 16-wide tile (column
 // n = 8 (r % 2) + f), then X1 = S [W_l] + Esum b_l from a per-wave LDS copy of
 // S, Esum[j] = sum_p Ephi[j][p] (the DFT of the constant input, host-summed).
 // Needs P % 16 == 0, J == 32, NIN == 8 and 64 % C == 0.
 constexpr int kLiftWaveJ = 32;
-constexpr int kLiftRows = 4;
 
-template <int NIN>
+template <int NIN, int ROWS>
 __global__ __launch_bounds__(256) void lift_dft_wave_kernel(const float* __restrict__ in, const float* __restrict__ Ephi,
                                                             const float* __restrict__ Esum,
                                                             const float* __restrict__ Wl, const float* __restrict__ bl,
                                                             float* __restrict__ X1, int P, int C, long long rows) {
     static_assert(NIN == 8, "two rows' inputs fill one 16-wide tile");
     constexpr int SW = NIN + 1;                           // padded row of S in LDS
-    constexpr int J = kLiftWaveJ, JT = J / 16, RT = kLiftRows / 2;
-    __shared__ float s_S[4][kLiftRows][J * SW];
+    constexpr int J = kLiftWaveJ, JT = J / 16, RT = ROWS / 2;
+    __shared__ float s_S[4][ROWS][J * SW];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int mr = lane & 15, g = lane >> 4;
-    const long long row0 = (blockIdx.x * 4LL + wave) * kLiftRows;
+    const long long row0 = (blockIdx.x * 4LL + wave) * ROWS;
     if (row0 >= rows) return;                             // no barrier below: waves are independent
-    const int nr = static_cast<int>(rows - row0 < kLiftRows ? rows - row0 : kLiftRows);
+    const int nr = static_cast<int>(rows - row0 < ROWS ? rows - row0 : ROWS);
     const int P4 = P >> 2;
     f32x4 acc[RT][JT];
 #pragma unroll
@@ -854,8 +861,18 @@ __global__ __launch_bounds__(256) void column_sum_kernel(const float* part, long
     const int tx = threadIdx.x & 31, rl = threadIdx.x >> 5;
     const int j = blockIdx.x * 32 + tx;
     Kahan s;
-    if (j < cols)
-        for (long long r = rl; r < rows; r += 8) s.add(part[r * cols + j]);
+    if (j < cols) {
+        // eight rows' loads are issued before their adds
+        long long r = rl;
+        for (; r + 56 < rows; r += 64) {
+            float v[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v[q] = part[(r + 8 * q) * cols + j];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) s.add(v[q]);
+        }
+        for (; r < rows; r += 8) s.add(part[r * cols + j]);
+    }
     __shared__ float red[8][32];
     red[rl][tx] = s.value();
     __syncthreads();
@@ -885,6 +902,274 @@ __global__ __launch_bounds__(256) void column_partial_kernel(const float* x, lon
         Kahan t;
         for (int q = 0; q < per; ++q) t.add(red[q * C + threadIdx.x]);
         partial[blockIdx.x * C + threadIdx.x] = t.value();
+    }
+}
+
+// ---- fused backward of a Fourier layer, one block per run of (bubble, theta) rows
+//
+// The adjoint of fno_row_kernel.  With dz_l the loss gradient at layer l's
+// pre-activations and X1' [rows][J][C] the gradient at its phi coefficients
+// (the adjoint theta stage's result), a grid row's gradient at the layer's input is
+//   dx = dz_l W_l^T + Ephi^T X1'            (one MFMA product with K = C + J),
+// which is the gradient at layer l - 1's output, so the same block goes on with
+//   dz = dx act'(z_{l-1})                   (stored)
+//   Z'  = Iphi^T dz                         (per row: input of layer l - 1's adjoint theta stage)
+//   dW += x_{l-1}^T dz, db += sum dz        (kept in registers over the block's rows,
+//                                            one partial per block)
+// Rows are independent but for the theta stage, so a layer is one launch and
+// dz is the only activation gradient in memory; x_0 is lifted from the input
+// features (x null).  MODE 0 (top): dx = dout Q^T of the projection instead,
+// whose own gradient dQ = x_L^T dout, dq = sum dout it also forms (FP32).
+// MODE 2 (bottom): dx is the gradient at the lifted features: dW_l = in^T dx,
+// db_l = sum dx, nothing else.
+// Operands are rounded to BF16 as gemm_kernel rounds them; the bias sums are
+// compensated FP32 of the unrounded values.
+//
+// What bounds it: 512 B per cell (dz, z, x in, dz out) of HBM traffic, 200 us
+// at 5.4 TB/s for 16 bubbles of 256 x 512 at width 32; measured 313 us (3.4
+// TB/s, latency: 128 registers allow four waves per SIMD; 428 us with one
+// block per CU).  It replaces, per layer, act_grad (148 us), three passes for
+// the bias and weight gradients (183 + 18 + 300 us) and three row GEMMs of 300
+// us each: a training window's backward pass went from 7.5 to 1.6 ms.
+constexpr int kBackUnroll = 1;
+enum { kBackTop = 0, kBackMid = 1, kBackBottom = 2 };
+
+struct RowBackArgs {
+    const float* dz;                // [rows][P][C] of layer l (mid, bottom); dz_out may be the same array
+    const float* X1;                // [rows][J][C] (mid, bottom)
+    const float* W;                 // [C][C] of layer l (mid, bottom)
+    const unsigned short* EphiT;    // [P][J] BF16
+    const unsigned short* IphiT;    // [J][P] BF16
+    const float* z;                 // [rows][P][C] pre-activations of layer l - 1 (mid)
+    const float* x;                 // [rows][P][C] input of layer l - 1; null: lifted from `in`
+    const float* in;                // [rows][P][kLiftIn]
+    const float* Wl;                // [kLiftIn][C]
+    const float* bl;                // [C]
+    const float* xL;                // [rows][P][C] output of the last layer (top)
+    const float* dout;              // [rows][P][kProjOut] (top)
+    const float* Q;                 // [C][kProjOut] (top)
+    float* dz_out;                  // [rows][P][C] (top, mid)
+    float* Z_out;                   // [rows][J][C] (top, mid)
+    float* part;                    // [blocks][C C + C] weight and bias partials ([kLiftIn C + C] at the bottom)
+    float* part_q;                  // [blocks][C kProjOut + kProjOut] (top)
+    int rows;
+};
+
+template <int RT, int CT, int JT, int WAVES, int MODE>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4, 8))) void fno_row_back_kernel(const RowBackArgs a) {
+    constexpr int C = 16 * CT, J = 16 * JT, K = C + J, P = 16 * RT * WAVES, NT = 64 * WAVES;
+    constexpr int MT = MODE == kBackBottom ? 1 : CT;          // 16-row tiles of the weight gradient
+    constexpr int MR = MODE == kBackBottom ? kLiftIn : C;     // its rows
+    constexpr int REDW = (J > C ? J : C) * C;
+    __shared__ unsigned short Bs[C][K + 4];                   // [input channel][k]: W_l^T, then X1'
+    __shared__ float red[WAVES][REDW];
+    __shared__ float s_lift[(kLiftIn + 1) * C];               // W_l rows, then b_l
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int mr = lane & 15, kq = 4 * (lane >> 4);
+    if (MODE != kBackTop)
+        for (int q = threadIdx.x; q < C * C; q += NT) Bs[q / C][q % C] = to_bf16(a.W[q]);
+    const bool lift = MODE != kBackBottom && a.x == nullptr;
+    if (lift)
+        for (int q = threadIdx.x; q < (kLiftIn + 1) * C; q += NT)
+            s_lift[q] = q < kLiftIn * C ? a.Wl[q] : a.bl[q - kLiftIn * C];
+    if (lift && MODE == kBackTop) __syncthreads();            // mid: the row loop's first barrier
+    float qv[CT][kProjOut];
+    if (MODE == kBackTop)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int j = 0; j < kProjOut; ++j) qv[ct][j] = a.Q[(16 * ct + mr) * kProjOut + j];
+    f32x4 gw[MT][CT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) gw[mt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+    Kahan gb[CT], gq[CT][kProjOut], gqb[kProjOut];
+
+    for (int row = blockIdx.x; row < a.rows; row += gridDim.x) {
+        const long long r0 = static_cast<long long>(row) * P;
+        if (MODE != kBackTop) {
+            const float* X1 = a.X1 + static_cast<long long>(row) * J * C;
+            for (int q = threadIdx.x; q < J * C; q += NT) Bs[q % C][C + q / C] = to_bf16(X1[q]);
+            __syncthreads();
+        }
+        f32x4 accZ[JT][CT];
+#pragma unroll
+        for (int jt = 0; jt < JT; ++jt)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) accZ[jt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // Rolled: unrolled, the loads of all row tiles take 200 registers.
+#pragma unroll kBackUnroll
+        for (int rt = 0; rt < RT; ++rt) {
+            const int p0 = (wave * RT + rt) * 16;
+            // ---- dx of cells p0 .. p0 + 15: lane (mr, g) holds cells 4 g + v, channel 16 ct + mr
+            f32x4 acc[CT];
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) acc[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (MODE == kBackTop) {
+                float q4[CT][kProjOut] = {};
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const long long c = r0 + p0 + kq + v;
+                    const float2 d = *reinterpret_cast<const float2*>(a.dout + c * kProjOut);
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct) {
+                        acc[ct][v] = fmaf(d.y, qv[ct][1], d.x * qv[ct][0]);
+                        const float xl = a.xL[c * C + 16 * ct + mr];
+                        q4[ct][0] = fmaf(xl, d.x, q4[ct][0]);
+                        q4[ct][1] = fmaf(xl, d.y, q4[ct][1]);
+                    }
+                    if (mr == 0) {
+                        gqb[0].add(d.x);
+                        gqb[1].add(d.y);
+                    }
+                }
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                    for (int j = 0; j < kProjOut; ++j) gq[ct][j].add(q4[ct][j]);
+            } else {
+#pragma unroll
+                for (int ks = 0; ks < CT; ++ks) {
+                    const float4 v = *reinterpret_cast<const float4*>(a.dz + (r0 + p0 + mr) * C + ks * 16 + kq);
+                    const bf16x4 A = bf16x4{static_cast<short>(to_bf16(v.x)), static_cast<short>(to_bf16(v.y)),
+                                            static_cast<short>(to_bf16(v.z)), static_cast<short>(to_bf16(v.w))};
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct) {
+                        const bf16x4 B = *reinterpret_cast<const bf16x4*>(&Bs[ct * 16 + mr][ks * 16 + kq]);
+                        acc[ct] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A, B, acc[ct], 0, 0, 0);
+                    }
+                }
+#pragma unroll
+                for (int js = 0; js < JT; ++js) {
+                    const bf16x4 A = *reinterpret_cast<const bf16x4*>(a.EphiT + (p0 + mr) * J + js * 16 + kq);
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct) {
+                        const bf16x4 B = *reinterpret_cast<const bf16x4*>(&Bs[ct * 16 + mr][C + js * 16 + kq]);
+                        acc[ct] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A, B, acc[ct], 0, 0, 0);
+                    }
+                }
+            }
+            // ---- through the activation of layer l - 1; stores and sums
+            bf16x4 Bd[CT];
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const long long e = (r0 + p0 + kq + v) * C + 16 * ct + mr;
+                    float d = acc[ct][v];
+                    if (MODE == kBackMid) d *= gelu_exp_grad(a.z[e]);
+                    if (MODE != kBackBottom) a.dz_out[e] = d;
+                    gb[ct].add(d);
+                    Bd[ct][v] = static_cast<short>(to_bf16(d));
+                }
+            }
+            // ---- weight gradient: A[m][k] = x[cell 4 g + v][m]
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                bf16x4 A;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const long long c = r0 + p0 + kq + v;
+                    float xv;
+                    if (MODE == kBackBottom) {
+                        xv = mr < kLiftIn ? a.in[c * kLiftIn + mr] : 0.f;
+                    } else if (lift) {
+                        const float4 f0 = *reinterpret_cast<const float4*>(a.in + c * kLiftIn);
+                        const float4 f1 = *reinterpret_cast<const float4*>(a.in + c * kLiftIn + 4);
+                        const float f[kLiftIn] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
+                        xv = s_lift[kLiftIn * C + 16 * mt + mr];
+#pragma unroll
+                        for (int i = 0; i < kLiftIn; ++i) xv = fmaf(f[i], s_lift[i * C + 16 * mt + mr], xv);
+                    } else {
+                        xv = a.x[c * C + 16 * mt + mr];
+                    }
+                    A[v] = static_cast<short>(to_bf16(xv));
+                }
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct)
+                    gw[mt][ct] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A, Bd[ct], gw[mt][ct], 0, 0, 0);
+            }
+            // ---- Z'[j][c] += Iphi[p][j] dz[p][c]
+            if (MODE != kBackBottom) {
+#pragma unroll
+                for (int jt = 0; jt < JT; ++jt) {
+                    const bf16x4 A = *reinterpret_cast<const bf16x4*>(a.IphiT + (jt * 16 + mr) * P + p0 + kq);
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct)
+                        accZ[jt][ct] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A, Bd[ct], accZ[jt][ct], 0, 0, 0);
+                }
+            }
+        }
+        if (MODE != kBackBottom) {
+#pragma unroll
+            for (int jt = 0; jt < JT; ++jt)
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) red[wave][(jt * 16 + kq + v) * C + ct * 16 + mr] = accZ[jt][ct][v];
+        }
+        __syncthreads();                       // Bs is read, red written
+        if (MODE != kBackBottom) {
+            float* Z = a.Z_out + static_cast<long long>(row) * J * C;
+            for (int q = threadIdx.x; q < J * C; q += NT) {
+                float sum = 0.f;
+#pragma unroll
+                for (int w = 0; w < WAVES; ++w) sum += red[w][q];
+                Z[q] = sum;
+            }
+            if (MODE == kBackTop) __syncthreads();             // red is read (mid: the next row's first barrier)
+        }
+    }
+    // ---- the block's partials: waves folded in order
+    __syncthreads();
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                if (mt * 16 + kq + v < MR) red[wave][(mt * 16 + kq + v) * C + ct * 16 + mr] = gw[mt][ct][v];
+    __syncthreads();
+    constexpr int COLS = MR * C + C;
+    float* part = a.part + static_cast<long long>(blockIdx.x) * COLS;
+    for (int q = threadIdx.x; q < MR * C; q += NT) {
+        float sum = 0.f;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) sum += red[w][q];
+        part[q] = sum;
+    }
+    __syncthreads();
+    // bias (and projection) sums: the four lane groups' values of a channel, wave by wave
+    constexpr int NB = MODE == kBackTop ? 1 + kProjOut : 1;
+    static_assert(4 * NB * C + 4 * kProjOut <= REDW, "sums fit the wave's LDS slice");
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+        red[wave][(kq / 4) * C + ct * 16 + mr] = gb[ct].value();
+        if (MODE == kBackTop)
+#pragma unroll
+            for (int j = 0; j < kProjOut; ++j)
+                red[wave][(4 * (1 + j) + kq / 4) * C + ct * 16 + mr] = gq[ct][j].value();
+    }
+    if (MODE == kBackTop && mr == 0)
+#pragma unroll
+        for (int j = 0; j < kProjOut; ++j) red[wave][4 * NB * C + 4 * j + kq / 4] = gqb[j].value();
+    __syncthreads();
+    for (int q = threadIdx.x; q < NB * C; q += NT) {
+        const int k = q / C, c = q - k * C;
+        Kahan t;
+        for (int w = 0; w < WAVES; ++w)
+            for (int g = 0; g < 4; ++g) t.add(red[w][(4 * k + g) * C + c]);
+        if (k == 0)
+            part[MR * C + c] = t.value();
+        else
+            a.part_q[static_cast<long long>(blockIdx.x) * (C * kProjOut + kProjOut) + c * kProjOut + k - 1] = t.value();
+    }
+    if (MODE == kBackTop && threadIdx.x < kProjOut) {
+        Kahan t;
+        for (int w = 0; w < WAVES; ++w)
+            for (int g = 0; g < 4; ++g) t.add(red[w][4 * NB * C + 4 * threadIdx.x + g]);
+        a.part_q[static_cast<long long>(blockIdx.x) * (C * kProjOut + kProjOut) + C * kProjOut + threadIdx.x] = t.value();
     }
 }
 

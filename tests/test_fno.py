@@ -157,6 +157,40 @@ def test_gpu_fused_layers_match_reference():
     m.close()
 
 
+# The fused backward kernel at the corners of its shapes: every n_phi with one
+# and two channel and mode tiles, a single layer (the projection's and the
+# lift's gradients meet in one kernel), one grid row per block and, with more
+# rows than blocks (768 of 512), an uneven walk.
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_theta,n_phi,width,modes_theta,modes_phi,layers,batch", [
+    (32, 128, 32, 4, 8, 2, 1),
+    (32, 128, 16, 4, 16, 1, 2),
+    (16, 256, 16, 4, 8, 1, 1),
+    (16, 256, 32, 8, 16, 3, 3),
+    (48, 256, 32, 3, 8, 2, 1),
+    (8, 512, 32, 2, 16, 2, 1),
+    (8, 512, 16, 4, 16, 2, 3),
+    (256, 128, 16, 4, 8, 2, 3),
+])
+def test_gpu_fused_backward_shapes(n_theta, n_phi, width, modes_theta, modes_phi, layers, batch):
+    from soap_bubble_simulation_amd import _lib as L
+    from soap_bubble_simulation_amd.surrogate import FnoSurrogate
+    m = FnoSurrogate(n_theta=n_theta, n_phi=n_phi, width=width, modes_theta=modes_theta, modes_phi=modes_phi,
+                     layers=layers, window=4, max_batch=batch)
+    assert m.kernel_paths() & L.FNO_PATH_FUSED_ROWS
+    s = R.Shapes.of(m.config)
+    flat, x, t = rand_problem(s, batch, seed=31, scale=0.25)
+    f32, x32, t32 = flat.astype(np.float32), x.astype(np.float32), t.astype(np.float32)
+    m.set_params(f32)
+    rl, rg, _ = R.loss_and_grad(f32.astype(np.float64), x32.astype(np.float64), t32.astype(np.float64), s)
+    for _ in range(2):                      # the second call starts from used buffers
+        loss, g = m.gradient(x32, t32)
+        assert abs(loss - rl) <= 1e-2 * rl
+        for name, sl in group_slices(s):
+            assert rel(g[sl], rg[sl]) <= 2e-2, (name, rel(g[sl], rg[sl]))
+    m.close()
+
+
 @pytest.mark.gpu
 def test_gpu_train_step_reduces_loss(model):
     s = R.Shapes.of(model.config)
