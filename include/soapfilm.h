@@ -205,8 +205,12 @@ int sf_drainage_kernel_timing(sf_drainage* ctx, int32_t enable, double* avg_ms,
  * step per launch.  A launch of two steps never straddles a rebase (every
  * rebase_interval steps), so an odd step count or a rebase boundary gives
  * one one-step launch.  The default is 2 on grids of about 2 million cells
- * and more (1024 x 2048 and up), 1 below.  sf_drainage_get_steps_per_launch
- * returns what sf_drainage_step will use; sf_drainage_kernel_timing then
+ * and more (1024 x 2048 and up), 1 below.  On grids with n_phi <= 1024 and
+ * few rows (1500 x 1024, 4000 x 256) sf_drainage_step takes up to 8 steps
+ * per launch by itself, for all flags, with the same cell arithmetic and
+ * pole rows formed in FP64; setting 1 here switches that off.
+ * sf_drainage_get_steps_per_launch returns 1 or 2, what the launches of the
+ * streaming kernels take; sf_drainage_kernel_timing then
  * averages over all its launches, of one or two steps.
  * sf_drainage_step_spectral renders both states of a two-step launch: the
  * launch also writes the state between its steps.  No counterpart in the

@@ -148,6 +148,22 @@ __global__ __launch_bounds__(256) void diag_finalize_kernel(const double2* part,
                 pole_mass_fixed, hist, slot, red_d);
 }
 
+// The history entries of a drainage_multi_kernel launch: block k folds step
+// k's per-block partials (the pole rows are in them unless copied through).
+__global__ __launch_bounds__(64) void multi_diag_kernel(const double2* part, int nblocks, double fixed, double2* hist,
+                                                        int slot0, int cap) {
+    double m = 0.0, l = 0.0;
+    const double2* p = part + static_cast<size_t>(blockIdx.x) * nblocks;
+    for (int b = threadIdx.x; b < nblocks; b += 64) {
+        m += p[b].x;
+        l = fmax(l, p[b].y);
+    }
+    m = wave_dsum(m);
+    l = wave_dmax(l);
+    if (threadIdx.x == 0)
+        hist[(slot0 + static_cast<int>(blockIdx.x)) % cap] = make_double2(m + fixed, l > 0.0 ? 2.0 / l : INFINITY);
+}
+
 __global__ void fill_kernel(float* p, size_t n, float v) {
     const size_t c = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x;
     if (c < n) p[c] = v;
@@ -227,6 +243,17 @@ static StepFn step_fn(bool rebase, int gmode, bool marangoni, bool diag, bool ve
     return band[rebase][gmode][marangoni][diag];
 }
 
+using MultiFn = void (*)(const MultiArgs);
+
+static MultiFn multi_fn(int gmode, bool marangoni, bool diag) {
+    static const MultiFn tab[3][2][2] = {      // the Marangoni term reads Γ, frozen or not
+        {{&drainage_multi_kernel<0, false, false>, &drainage_multi_kernel<0, false, true>}, {nullptr, nullptr}},
+        {{nullptr, nullptr}, {&drainage_multi_kernel<1, true, false>, &drainage_multi_kernel<1, true, true>}},
+        {{&drainage_multi_kernel<2, false, false>, &drainage_multi_kernel<2, false, true>},
+         {&drainage_multi_kernel<2, true, false>, &drainage_multi_kernel<2, true, true>}}};
+    return tab[gmode][marangoni][diag];
+}
+
 // Two-step launches: [rebase][gmode 0 or 2][OPT].
 template <bool RB, int GM, int OPT>
 static void launch_band2(dim3 grid, dim3 block, hipStream_t s, hipEvent_t t0, hipEvent_t t1, const StepArgs& a) {
@@ -290,6 +317,9 @@ Drainage::Drainage(const sf_params& prm, int n_theta, int n_phi) : p(prm), nt(n_
         }
     }
     steps_per_launch = rows_per_block2 >= 4 ? 2 : 1;
+    // Small grids: several steps per launch in LDS, unless a kernel is forced
+    // or the caller sets the steps per launch.
+    if (!force && !std::getenv("SOAPFILM_ROWS_PER_BLOCK") && !std::getenv("SOAPFILM_ROWS_PER_BLOCK2")) multi_plan();
     if (const char* e = std::getenv("SOAPFILM_ROWS_PER_BLOCK2"))
         rows_per_block2 = std::min(std::max(1, std::atoi(e)), kBandMax);
     for (int k = 0; k < 2; ++k) {
@@ -318,12 +348,37 @@ Drainage::~Drainage() {
     }
     dfree(rows); dfree(rowd); dfree(diag_hist);
     for (int k = 0; k < kDiagBufs; ++k) dfree(diag_part[k]);
-    dfree(lo_mid); dfree(hpole_mid[0]); dfree(hpole_mid[1]);
+    dfree(multi_part); dfree(lo_mid); dfree(hpole_mid[0]); dfree(hpole_mid[1]);
     dfree(stats_part); dfree(stats_out); dfree(gather_idx); dfree(gather_out);
     dfree(rgb); dfree(cmf_dev); dfree(spec_rows); dfree(spec_cols); dfree(spec_view); dfree(caustic);
     step_timer.destroy();
     spec_timer.destroy();
     if (stream) (void)hipStreamDestroy(stream);
+}
+
+// Rows per block and steps per launch of drainage_multi_kernel for this grid
+// (multi_steps 0: not used).  One block per CU at most.  A launch costs its
+// gap, the load and the store, a step a latency floor and the rows it updates,
+// of which every further step adds two: sqrt(10^4 / n_phi) steps were best, or
+// within 4 % of the best, from half to twice that number.  Against the
+// streaming kernels, us per step (thinning alone | surfactant, thinning and
+// diagnostics): 64 x 128 4.9 -> 2.7 | 6.3 -> 3.7, 256 x 512 5.2 -> 3.3 | 7.5 ->
+// 5.3, 64 x 1024 5.6 -> 4.6 | 7.6 -> 6.7, 1500 x 1024 7.5 -> 7.0 | 12.7 -> 12.0.
+// Longer rows leave too little to a step beside the copies: 40 x 1500 6.2 ->
+// 6.7 | 7.9 -> 9.2, hence kMultiMaxCols.
+void Drainage::multi_plan() {
+    constexpr int kCus = 256;
+    constexpr size_t kLdsBytes = 150 * 1024;
+    if (nt < 3 || np > kMultiMaxCols) return;
+    multi_rows = (nt - 2 + kCus - 1) / kCus;
+    if (multi_rows > kMultiRows) return;
+    int k = static_cast<int>(std::lround(std::sqrt(1e4 / np)));
+    k = std::max(2, std::min(k, kMultiSteps));
+    for (; k >= 2; --k) {
+        const size_t held = static_cast<size_t>(multi_rows + 2 * k) * np;
+        if (held * 12 <= kLdsBytes && held - 2 * np <= static_cast<size_t>(kMultiCells) * kMultiThreads) break;
+    }
+    multi_steps = k >= 2 ? k : 0;
 }
 
 // Per-row coefficient tables, FP64 on the host then rounded (drainage.rs:315-324).
@@ -762,11 +817,97 @@ void Drainage::launch_two(double dt, bool with_mid) {
     steps_taken += 2;
 }
 
+// k steps in one launch of drainage_multi_kernel (2 <= k <= multi_steps).
+void Drainage::launch_multi(double dt, int k) {
+    const bool marangoni = (p.flags & SF_FLAG_MARANGONI) != 0;
+    const bool surfactant = (p.flags & SF_FLAG_SURFACTANT) != 0;
+    const int gmode = surfactant ? 2 : (marangoni ? 1 : 0);
+    const bool diag = (p.flags & SF_FLAG_DIAG) != 0;
+    const bool h_avg = !(p.flags & SF_FLAG_POLES_COPY_H);
+    const bool g_avg = surfactant && (p.flags & SF_FLAG_POLES_AVG_GAMMA);
+    const int rebase_every = p.rebase_interval > 0 ? static_cast<int>(p.rebase_interval) : 1;
+    const unsigned blocks = cdiv(nt - 2, multi_rows);
+    MultiArgs m{};
+    fill_common_args(m.s, static_cast<float>(dt));
+    m.steps = k;
+    m.rows = multi_rows;
+    m.inv_np = 1.0 / np;
+    for (int s = 0; s < k; ++s) {
+        StepArgs one{};
+        schedule_fronts(dt, one);
+        m.nf[s] = one.nfronts;
+        for (int f = 0; f < one.nfronts; ++f) m.fr[s][f] = one.fr[f];
+        if (one.nfronts > 0) {
+            m.s.tfe_g_hi = one.tfe_g_hi;
+            m.s.tfe_g_lo = one.tfe_g_lo;
+        }
+        last_boxes.assign(one.fr, one.fr + one.nfronts);
+        current_time += dt;
+        if (since_rebase + 1 >= rebase_every) {
+            m.rebase |= 1u << s;
+            since_rebase = 0;
+        } else {
+            ++since_rebase;
+        }
+    }
+    StepArgs& a = m.s;
+    a.hi_in = hi[cur_hi];
+    a.lo_in = lo[cur];
+    a.g_in = g[cur_g];
+    a.hi_out = hi[1 - cur_hi];
+    a.lo_out = lo[1 - cur];
+    a.g_out = g[1 - cur_g];
+    a.h_pole_mean = (poles_virtual && h_avg) ? 1 : 0;
+    a.g_pole_mean = (poles_virtual && g_avg) ? 1 : 0;
+    a.h_pole_sum = h_avg ? 1 : 0;
+    a.g_pole_sum = g_avg ? 1 : 0;
+    a.hpole_in = hpole[cur_pole];
+    a.gpole_in = gpole[cur_pole];
+    a.hpole_out = hpole[1 - cur_pole];
+    a.gpole_out = gpole[1 - cur_pole];
+    finalize_diag();
+    if (diag && !multi_part) multi_part = dalloc<double2>(static_cast<size_t>(kMultiSteps) * blocks);
+    m.part = multi_part;
+    const size_t bytes = static_cast<size_t>(multi_rows + 2 * k) * np * (gmode ? 12 : 8);
+    const MultiFn fn = multi_fn(gmode, marangoni, diag);
+    if (bytes > 64 * 1024)
+        SF_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   static_cast<int>(bytes)));
+    if (step_timer.enabled) {
+        auto& ev = step_timer.next(stream);
+        hipExtLaunchKernelGGL(fn, dim3(blocks), dim3(kMultiThreads), bytes, stream, ev.first, ev.second, 0, m);
+    } else {
+        hipLaunchKernelGGL(fn, dim3(blocks), dim3(kMultiThreads), bytes, stream, m);
+    }
+    SF_HIP(hipGetLastError());
+    if (diag) {
+        hipLaunchKernelGGL(multi_diag_kernel, dim3(k), dim3(64), 0, stream, multi_part, static_cast<int>(blocks),
+                           h_avg ? 0.0 : pole_mass_fixed, diag_hist, static_cast<int>(hist_count % kHistCap),
+                           static_cast<int>(kHistCap));
+        SF_HIP(hipGetLastError());
+        hist_count += k;
+    }
+    cur = 1 - cur;
+    if (surfactant) cur_g = 1 - cur_g;
+    if (m.rebase) cur_hi = 1 - cur_hi;
+    if (h_avg || g_avg) {
+        cur_pole = 1 - cur_pole;
+        poles_virtual = true;
+    }
+    steps_taken += k;
+}
+
 void Drainage::step(int n_steps, double dt, bool flush) {
     if (tables_dirty) upload_tables();
     dt = resolve_dt(dt);
     for (int s = 0; s < n_steps;) {
-        if (two_step_next(n_steps - s)) {
+        const int left = n_steps - s;
+        if (multi_steps && left >= 2) {
+            // equal shares: 10 steps at 8 per launch go as 5 + 5
+            const int launches = (left + multi_steps - 1) / multi_steps, k = (left + launches - 1) / launches;
+            launch_multi(dt, k);
+            s += k;
+        } else if (two_step_next(n_steps - s)) {
             launch_two(dt, false);
             s += 2;
         } else {
@@ -1319,6 +1460,7 @@ extern "C" int sf_drainage_set_steps_per_launch(sf_drainage* ctx, int32_t steps)
         SF_REQUIRE(ctx != nullptr, SF_ERR_INVALID, "ctx is NULL");
         SF_REQUIRE(steps == 1 || steps == 2, SF_ERR_INVALID, "steps per launch must be 1 or 2, got %d", steps);
         D(ctx)->steps_per_launch = steps;
+        D(ctx)->multi_steps = 0;
     });
 }
 

@@ -66,6 +66,10 @@ struct Drainage {
     // steps_per_launch 2 asks for it, 1 keeps one step per launch.
     int steps_per_launch = 1;
     int rows_per_block2 = 16;     // band height of the two-step kernel
+    // Several steps per launch on small grids (drainage_multi_kernel): rows
+    // per block and the most steps, 0 where it is not used.
+    int multi_rows = 1, multi_steps = 0;
+    double2* multi_part = nullptr;
 
     // device state (see drainage_kernels.hpp for the layout)
     float* hi[2] = {nullptr, nullptr};
@@ -178,6 +182,8 @@ struct Drainage {
     // state between them).  dt is resolved; tables are uploaded.
     void launch_one(double dt);
     void launch_two(double dt, bool with_mid);
+    void multi_plan();
+    void launch_multi(double dt, int k);
     // The state between the steps of the last two-step launch made with
     // with_mid: high word, low word, ring partials.
     const float* mid_hi = nullptr;

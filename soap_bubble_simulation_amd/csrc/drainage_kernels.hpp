@@ -758,6 +758,312 @@ __device__ __forceinline__ void cell_step(const StepArgs& a, const RowF& rc, flo
     }
 }
 
+// ---------------------------------------------------------------------------
+// Several steps per launch on small grids, the state held in LDS.
+//
+// A one-step launch on a small grid is all latency: 5.0 us at 128 x 256 for
+// 0.05 us of arithmetic.  Here a block owns rows [r0, r1) with all their
+// columns, loads `steps` more rows on each side into LDS and advances them
+// `steps` times, each step updating one row less on each side, so that its
+// own rows are right at the end; only those are written back.  With whole
+// rows in a block the ring mean of a pole is formed inside it, by every
+// block whose rows reach the ring.  Any n_phi; every flag of the one-step
+// kernel.
+//
+// A step costs a latency floor of about 1.7 us (neighbours from LDS, two
+// barriers, the ring's tree) and then one CU's vector ALU ((r + steps - 1)
+// n_phi cells per block, about 75 instructions each), so the host takes one
+// block per CU or fewer rows, and fewer steps the wider the rows
+// (Drainage::multi_plan).  The ring sums are FP64 and go through DPP moves:
+// with LDS shuffles and a float-float tree they were 1 us of a step, front
+// boxes fetched per cell another 1 to 4 us.  us per step with thinning,
+// one-step launches -> these: 128 x 256 5.2 -> 3.4, 256 x 512 5.2 -> 3.3,
+// 500 x 1003 (no vector path) 13.5 -> 4.5.
+constexpr int kMultiSteps = 8;
+constexpr int kMultiThreads = 1024;
+constexpr int kMultiCells = 8;        // cells a thread updates per step, at most
+constexpr int kMultiMaxCols = 1024;   // longest row
+constexpr int kMultiRows = 16;        // rows a block owns, at most
+constexpr int kMultiRowsAll = kMultiRows + 2 * kMultiSteps;
+
+struct MultiArgs {
+    StepArgs s;
+    int steps;                        // 1 .. kMultiSteps
+    int rows;                         // rows a block owns, at most kMultiRows
+    unsigned rebase;                  // bit k: step k renormalises hi, lo
+    double inv_np;
+    int nf[kMultiSteps];
+    FrontBox fr[kMultiSteps][kMaxFronts];
+    double2* part;                    // diagnostics: [steps][blocks] {mass, max lambda}
+};
+
+// v of the lane that DPP control CTRL names added to v (0 where it names
+// none), on the vector ALU alone: the shuffles' LDS round trips would make up
+// most of a step here.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(b), CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), CTRL, ROWS, 0xf, false);
+    return v + __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned>(lo));
+}
+
+// Sum of each row of 16 lanes, in its lane 15 (row_shr 1, 2, 4, 8).
+__device__ __forceinline__ double row_sum(double v) {
+    v = dpp_add<0x111, 0xf>(v);
+    v = dpp_add<0x112, 0xf>(v);
+    v = dpp_add<0x114, 0xf>(v);
+    return dpp_add<0x118, 0xf>(v);
+}
+
+__device__ __forceinline__ double lane_value(double v, int lane) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane(static_cast<int>(b), lane);
+    const int hi = __builtin_amdgcn_readlane(static_cast<int>(b >> 32), lane);
+    return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned>(lo));
+}
+
+// Sum over the wave, uniform (row_bcast 15 and 31 carry the rows' sums on).
+__device__ __forceinline__ double wave_sum(double v) {
+    v = row_sum(v);
+    v = dpp_add<0x142, 0xa>(v);
+    v = dpp_add<0x143, 0xc>(v);
+    return lane_value(v, 63);
+}
+
+__device__ __forceinline__ float2 split_pair(double v) {
+    const float h = static_cast<float>(v);
+    return make_float2(h, static_cast<float>(v - static_cast<double>(h)));
+}
+
+template <int GMODE, bool MARANGONI, bool DIAG>
+__global__ __launch_bounds__(kMultiThreads) void drainage_multi_kernel(const MultiArgs m) {
+    constexpr bool GREAD = GMODE >= 1;
+    constexpr bool GWRITE = GMODE == 2;
+    constexpr int kWaves = kMultiThreads / 64, T = kMultiThreads;
+    const StepArgs& a = m.s;
+    extern __shared__ __align__(16) float lds_state[];
+    __shared__ float4 s_row[kMultiRowsAll];      // cot / (2 dth), 1 / (s^2 dph^2), dt coef sin, 1 / s
+    __shared__ double s_ring[4][kWaves];         // ring sums per wave: h top, h bottom, g top, g bottom
+    __shared__ RowD s_rowd[DIAG ? kMultiRows : 1];
+    __shared__ double s_mass[DIAG ? kMultiSteps : 1][kWaves], s_lam[DIAG ? kMultiSteps : 1][kWaves];
+    const int np = a.np, nt = a.nt, tid = threadIdx.x;
+    const int lane = tid & 63, wave = tid >> 6;
+    const int r0 = 1 + static_cast<int>(blockIdx.x) * m.rows, r1 = min(r0 + m.rows, nt - 1);
+    const int e0 = max(r0 - m.steps, 0), e1 = min(r1 + m.steps, nt);
+    const int cells = (e1 - e0) * np;
+    float2* HL = reinterpret_cast<float2*>(lds_state);       // (hi, lo) of the block's rows
+    float* G = lds_state + 2 * cells;
+    {
+        const size_t base = static_cast<size_t>(e0) * np;
+        for (int c = tid; c < cells; c += T) {
+            HL[c] = make_float2(a.hi_in[base + c], a.lo_in[base + c]);
+            if (GREAD) G[c] = a.g_in[base + c];
+        }
+    }
+    if (tid < e1 - e0) {
+        const RowF rc = a.rows[e0 + tid];
+        s_row[tid] = make_float4(rc.cot * a.inv_2dth, rc.inv_s2 * a.inv_dph2, a.dt * a.coef * rc.sin_t, rc.inv_s);
+    }
+    if (DIAG && tid < r1 - r0) s_rowd[tid] = a.rowd[r0 + tid];
+    // Pole rows: the previous launch's ring sums (mean), or the rows as they
+    // are in the first step, and this launch's ring sums after it.
+    float2 mean[2] = {make_float2(0.f, 0.f), make_float2(0.f, 0.f)};
+    float gmean[2] = {0.f, 0.f};
+    bool have = a.h_pole_mean != 0, ghave = GREAD && a.g_pole_mean != 0;
+    for (int e = 0; e < 2; ++e) {
+        if (e == 0 ? e0 != 0 : e1 != nt) continue;
+        if (have) mean[e] = pole_mean(a.hpole_in + e * a.ntiles, a.ntiles, a.np_f);
+        if (ghave) {
+            const float2 g = pole_mean(a.gpole_in + e * a.ntiles, a.ntiles, a.np_f);
+            gmean[e] = g.x + g.y;
+        }
+    }
+    double total[2] = {0.0, 0.0}, gtotal[2] = {0.0, 0.0};
+    // A thread's cells lie T apart in the step's rows; row and column of each
+    // relative to the first row are the same in every step.
+    int rel[kMultiCells], col[kMultiCells];
+    rel[0] = tid / np;
+    col[0] = tid - rel[0] * np;
+    const int dr = T / np, dc = T - dr * np;
+#pragma unroll
+    for (int q = 1; q < kMultiCells; ++q) {
+        rel[q] = rel[q - 1] + dr;
+        col[q] = col[q - 1] + dc;
+        if (col[q] >= np) {
+            col[q] -= np;
+            ++rel[q];
+        }
+    }
+    const float G0 = a.inv_dth2, dtD = a.dt * a.d_r2;
+    __syncthreads();
+    for (int k = 0; k < m.steps; ++k) {
+        const int left = m.steps - 1 - k;
+        const int u0 = max(1, r0 - left), u1 = min(nt - 1, r1 + left);      // rows updated in this step
+        const int count = (u1 - u0) * np, first = (u0 - e0) * np;
+        const bool rebase = (m.rebase >> k) & 1;
+        const bool cap = u0 == 1 || u1 == nt - 1;      // the step meets a ring
+        // Bit q: cell q lies in a front.  Front by front, so that a box is
+        // fetched once per step and skipped where the block's rows miss it.
+        unsigned front = 0;
+        const int nf = m.nf[k];
+#pragma unroll 4
+        for (int f = 0; f < nf; ++f) {
+            const FrontBox b = m.fr[k][f];
+            if (b.ihi < u0 || b.ilo >= u1) continue;
+#pragma unroll
+            for (int q = 0; q < kMultiCells; ++q) {
+                if (q * T >= count) break;
+                const int i = u0 + rel[q];
+                int d = col[q] - b.j0;
+                if (d < 0) d += np;
+                front |= static_cast<unsigned>(i >= b.ilo && i <= b.ihi && d < b.len) << q;
+            }
+        }
+        float2 nhl[kMultiCells];
+        float ng[kMultiCells];
+        double ring[2] = {0.0, 0.0}, gring[2] = {0.0, 0.0};
+        double mass = 0.0, lam = 0.0;
+#pragma unroll
+        for (int q = 0; q < kMultiCells; ++q) {
+            if (q * T >= count) break;                                      // uniform
+            const bool in = tid + q * T < count;
+            // out of range: the first cell again, not stored
+            const int c = in ? first + tid + q * T : first, i = in ? u0 + rel[q] : u0, j = in ? col[q] : 0;
+            const int w = j == 0 ? c + np - 1 : c - 1, e = j + 1 == np ? c - np + 1 : c + 1;
+            const float4 rw = s_row[i - e0];
+            const float2 C = HL[c], Wv = HL[w], Ev = HL[e];
+            float2 N = HL[c - np], S = HL[c + np];
+            float cg = 0.f, gn = 0.f, gs = 0.f, gw = 0.f, ge = 0.f;
+            if (GREAD) {
+                cg = G[c];
+                gn = G[c - np];
+                gs = G[c + np];
+                gw = G[w];
+                ge = G[e];
+            }
+            if (cap) {
+                if (have && i == 1) N = mean[0];
+                if (have && i == nt - 2) S = mean[1];
+                if (GREAD && ghave && i == 1) gn = gmean[0];
+                if (GREAD && ghave && i == nt - 2) gs = gmean[1];
+            }
+            RowF rc{};
+            rc.inv_s = rw.w;
+            float lo_new, g_new;
+            cell_step<GMODE, MARANGONI>(a, rc, G0, rw.x, rw.y, dtD, rw.z, C.x, C.y, N.x, N.y, S.x, S.y, Wv.x, Wv.y, Ev.x,
+                                        Ev.y, cg, gn, gs, gw, ge, lo_new, g_new);
+            // ring values before the fronts act (update_poles runs first)
+            if (cap && in) {
+                const double hv = static_cast<double>(C.x) + static_cast<double>(lo_new);
+                if (i == 1) {
+                    ring[0] += hv;
+                    gring[0] += static_cast<double>(g_new);
+                }
+                if (i == nt - 2) {
+                    ring[1] += hv;
+                    gring[1] += static_cast<double>(g_new);
+                }
+            }
+            if (in && ((front >> q) & 1)) lo_new = front_thin(a, C.x, lo_new);
+            nhl[q] = make_float2(C.x, lo_new);
+            if (rebase) two_sum(C.x, lo_new, nhl[q].x, nhl[q].y);
+            ng[q] = g_new;
+            if (DIAG && in && i >= r0 && i < r1) {
+                const RowD& rd = s_rowd[i - r0];
+                const double hv = static_cast<double>(C.x) + static_cast<double>(lo_new);
+                mass += hv * rd.area;
+                lam = fmax(lam, rd.lam_grid + a.coef3 * rd.sin_abs * hv * hv);
+            }
+        }
+        __syncthreads();                         // every neighbour is read
+#pragma unroll
+        for (int q = 0; q < kMultiCells; ++q) {
+            if (q * T >= count) break;
+            if (tid + q * T < count) {
+                HL[first + tid + q * T] = nhl[q];
+                if (GWRITE) G[first + tid + q * T] = ng[q];
+            }
+        }
+        if (cap) {
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                if (a.h_pole_sum) {
+                    const double v = wave_sum(ring[e]);
+                    if (lane == 0) s_ring[e][wave] = v;
+                }
+                if (GWRITE && a.g_pole_sum) {
+                    const double v = wave_sum(gring[e]);
+                    if (lane == 0) s_ring[2 + e][wave] = v;
+                }
+            }
+        }
+        __syncthreads();                         // the new rows and the waves' ring sums are written
+        if (cap) {
+            // every wave folds the waves' sums (kWaves == 16 lanes); read here,
+            // written again only past the next step's first barrier
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                if (e == 0 ? u0 != 1 : u1 != nt - 1) continue;
+                if (a.h_pole_sum) {
+                    total[e] = lane_value(row_sum(lane < kWaves ? s_ring[e][lane] : 0.0), kWaves - 1);
+                    double v = total[e] * m.inv_np;
+                    v = fma(fma(-v, static_cast<double>(np), total[e]), m.inv_np, v);
+                    mean[e] = split_pair(v);
+                }
+                if (GWRITE && a.g_pole_sum) {
+                    gtotal[e] = lane_value(row_sum(lane < kWaves ? s_ring[2 + e][lane] : 0.0), kWaves - 1);
+                    gmean[e] = static_cast<float>(gtotal[e] * m.inv_np);
+                }
+            }
+        }
+        have = have || a.h_pole_sum;
+        ghave = ghave || (GWRITE && a.g_pole_sum);
+        if (DIAG) {
+            mass = wave_sum(mass);
+            lam = wave_dmax(lam);
+            if (lane == 0) {
+                if (a.h_pole_sum && wave == 0) {     // the owner of a ring adds its pole row
+                    if (r0 == 1) mass += a.pole_area_top * total[0];
+                    if (r1 == nt - 1) mass += a.pole_area_bot * total[1];
+                }
+                s_mass[k][wave] = mass;
+                s_lam[k][wave] = lam;
+            }
+        }
+    }
+    {
+        const int from = (r0 - e0) * np, own = (r1 - r0) * np;
+        const size_t base = static_cast<size_t>(r0) * np;
+        for (int c = tid; c < own; c += T) {
+            const float2 v = HL[from + c];
+            if (m.rebase) a.hi_out[base + c] = v.x;
+            a.lo_out[base + c] = v.y;
+            if (GWRITE) a.g_out[base + c] = G[from + c];
+        }
+    }
+    // Ring sums for the next launch: the total in the first tile's place.
+    for (int e = 0; e < 2; ++e) {
+        if (e == 0 ? r0 != 1 : r1 != nt - 1) continue;
+        for (int t = tid; t < a.ntiles; t += T) {
+            if (a.h_pole_sum) a.hpole_out[e * a.ntiles + t] = t == 0 ? split_pair(total[e]) : make_float2(0.f, 0.f);
+            if (GWRITE && a.g_pole_sum)
+                a.gpole_out[e * a.ntiles + t] = t == 0 ? split_pair(gtotal[e]) : make_float2(0.f, 0.f);
+        }
+    }
+    if (DIAG) {
+        __syncthreads();
+        if (tid < m.steps) {
+            double ms = 0.0, l = 0.0;
+            for (int w = 0; w < kWaves; ++w) {
+                ms += s_mass[tid][w];
+                l = fmax(l, s_lam[tid][w]);
+            }
+            m.part[static_cast<size_t>(tid) * gridDim.x + blockIdx.x] = make_double2(ms, l);
+        }
+    }
+}
+
 // Band-streaming variant of drainage_vec4_kernel: the same row update on a
 // band of a.rows_per_block rows (up to kBandMax) streamed through a window of
 // five row buffers, so tall bands cost no extra registers and re-read only
