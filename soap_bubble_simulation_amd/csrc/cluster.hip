@@ -83,6 +83,12 @@ struct KSum {
     __device__ inline float value() const { return s - c; }
 };
 
+// Orders a wave's LDS writes before its lanes' reads of one another's values.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+}
+
 __device__ inline void pair_force_add(float4 a, float4 b, const Consts& c, float& fx, float& fy, float& fz) {
 #pragma clang fp contract(off)
     const float dx = b.x - a.x, dy = b.y - a.y, dz = b.z - a.z;
@@ -104,23 +110,42 @@ __device__ inline void pair_force_add(float4 a, float4 b, const Consts& c, float
     fz += dz * inv * m;
 }
 
-// Partner positions of a run are loaded once per 64, one per lane, and
-// broadcast with v_readlane (the contact kernels).  Every lane of a wave
-// takes part (lanes past the last bubble load a clamped index and write
-// nothing), so each broadcast reads a loaded value.
-__device__ inline float4 lane_bcast(const float4& v, int t) {
-    return make_float4(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(v.x), t)),
-                       __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v.y), t)),
-                       __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v.z), t)),
-                       __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v.w), t)));
+// Bit t: partner q[t] may be nearer to a than ka a.w + kb b.w (all partners
+// but those clearly beyond: a 1e-5 margin on the square covers the rounding;
+// a NaN distance sets the bit).  Branch-free over kNear records fetched by
+// wide scalar loads (q is uniform), 10 vector instructions a pair: with the
+// test as a branch around the pair's terms nearly every one of the branches
+// was taken for some lane of the wave, each at the full cost of the terms.
+// Reads all kNear records, uses cnt <= kNear of them: the state arrays are
+// that much longer than the bubbles they hold.
+constexpr int kNear = 16;
+__device__ __forceinline__ unsigned near_mask(const float4* __restrict__ q, float4 a, int cnt, float ka, float kb) {
+    constexpr float kWide = 1.000006f;
+    ka *= kWide;
+    kb *= kWide;
+    const float ra = ka * a.w;
+    float4 b[kNear];
+#pragma unroll
+    for (int t = 0; t < kNear; ++t) b[t] = q[t];
+    unsigned mask = 0;
+#pragma unroll
+    for (int t = 0; t < kNear; ++t) {
+        const float dx = b[t].x - a.x, dy = b[t].y - a.y, dz = b[t].z - a.z;
+        const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz)), r = fmaf(kb, b[t].w, ra);
+        mask |= (d2 > r * r ? 0u : 1u) << t;
+    }
+    return mask & ((1u << cnt) - 1u);
 }
 
 // One partial per (block row, bubble): the block's kPairRuns runs are folded
-// in run order through LDS.  The partner index is wave-uniform, so partner
-// records come through scalar loads and cost the vector ALU nothing.
+// in run order through LDS.  A lane visits the partners of its own mask, in
+// order, from the wave's copy in LDS: two or three visits a wave and chunk at
+// cluster densities.  Issue-bound, half of it by the masks (n^2 pairs, 10
+// instructions): n = 4096 14.5 us with a branch a pair, 11.3 now.
 __global__ __launch_bounds__(64 * kPairRuns) void cluster_pair_kernel(const float4* __restrict__ pr, Consts c,
                                                                      float* __restrict__ part) {
     __shared__ float s_f[kPairRuns][3][kTile];
+    __shared__ float4 s_p[kPairRuns][kNear];
     const int lane = threadIdx.x & 63;
     const int w = threadIdx.x >> 6;
     const int run = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.y) * kPairRuns + w);
@@ -131,19 +156,23 @@ __global__ __launch_bounds__(64 * kPairRuns) void cluster_pair_kernel(const floa
     if (run < c.npruns) {                // whole wave
         const float4 a = pr[i < c.n ? i : c.n - 1];
         const int j0 = run * c.prun, j1 = min(c.n, j0 + c.prun);
-        for (int j = j0; j < j1; ++j) pair_force_add(a, pr[j], c, fx, fy, fz);
+        for (int j = j0; j < j1; j += kNear) {
+            const float4 mine = pr[j + (lane & (kNear - 1))];
+            unsigned mask = near_mask(pr + j, a, min(kNear, j1 - j), 3.f, 3.f);
+            if (lane < kNear) s_p[w][lane] = mine;
+            wave_lds_fence();
+            for (; mask; mask &= mask - 1) pair_force_add(a, s_p[w][__builtin_ctz(mask)], c, fx, fy, fz);
+            wave_lds_fence();
+        }
     }
     s_f[w][0][lane] = fx;
     s_f[w][1][lane] = fy;
     s_f[w][2][lane] = fz;
     __syncthreads();
-    if (w == 0 && i < c.n) {
-        float* dst = part + (static_cast<size_t>(blockIdx.y) * c.n + i) * 3;
-        for (int d = 0; d < 3; ++d) {
-            KSum k;
-            for (int r = 0; r < kPairRuns; ++r) k.add(s_f[r][d][lane]);
-            dst[d] = k.value();
-        }
+    if (w < 3 && i < c.n) {
+        KSum k;
+        for (int r = 0; r < kPairRuns; ++r) k.add(s_f[r][w][lane]);
+        part[(static_cast<size_t>(blockIdx.y) * c.n + i) * 3 + w] = k.value();
     }
 }
 
@@ -236,85 +265,151 @@ __device__ inline bool in_contact(float4 a, float4 b) {
     return (a.w + b.w - dist) > -a.w * kContactGap;
 }
 
+// Contacts (i, j > i) per partner run and bubble: count[run][i], and the first
+// coalescence candidate's key i n + j, else -1, in cand[run][i].  Tiles whose
+// partners all lie before them are skipped: n = 4096 25 -> 10 us with the
+// masks, cluster_connect_kernel 23 -> 8.
 __global__ __launch_bounds__(256) void cluster_contact_kernel(const float4* __restrict__ pr,
                                                               const float4* __restrict__ vt, Consts c,
                                                               int want_candidate, int* __restrict__ count,
                                                               long long* __restrict__ cand) {
 #pragma clang fp contract(off)
-    const int lane = threadIdx.x & 63;
-    const int run = blockIdx.y * kRunsPerBlock + (threadIdx.x >> 6);
+    __shared__ float4 s_p[kRunsPerBlock][kNear];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int run = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.y) * kRunsPerBlock + w);
     const int i = blockIdx.x * kTile + lane;
     if (run >= c.nruns) return;          // whole wave
-    const int ic = i < c.n ? i : c.n - 1;
-    const float4 a = pr[ic];
-    const float4 va = vt[ic];
     const int j0 = run * c.run, j1 = min(c.n, j0 + c.run);
     int k = 0;
     long long first = -1;
-    for (int jc = j0; jc < j1; jc += 64) {
-        const float4 mine = pr[min(jc + lane, c.n - 1)];
-        const int cnt = min(64, j1 - jc);
-        for (int t = 0; t < cnt; ++t) {
-            const int j = jc + t;
-            const float4 b = lane_bcast(mine, t);
-            if (j <= i || !in_contact(a, b)) continue;
-            ++k;
-            if (want_candidate && first < 0) {
-                // Weber number of the connection (foam_dynamics.rs:213-219).
-                const float dx = b.x - a.x, dy = b.y - a.y, dz = b.z - a.z;
-                const float dist = sqrtf(dx * dx + dy * dy + dz * dz);
-                const float nx = dx / dist, ny = dy / dist, nz = dz / dist;
-                const float4 vb = vt[j];
-                const float rel = (vb.x - va.x) * nx + (vb.y - va.y) * ny + (vb.z - va.z) * nz;
-                const float weber = c.density * (rel * rel) * a.w / c.surface_tension;
-                if (weber > c.coal_thr) first = static_cast<long long>(i) * c.n + j;
+    if (j1 > static_cast<int>(blockIdx.x) * kTile + 1) {      // some j > i
+        const float4 a = pr[i < c.n ? i : c.n - 1];
+        for (int jc = j0; jc < j1; jc += kNear) {
+            const float4 mine = pr[jc + (lane & (kNear - 1))];
+            unsigned mask = near_mask(pr + jc, a, min(kNear, j1 - jc), 1.3f, 1.f);
+            if (lane < kNear) s_p[w][lane] = mine;
+            wave_lds_fence();
+            for (; mask; mask &= mask - 1) {
+                const int t = __builtin_ctz(mask), j = jc + t;
+                const float4 b = s_p[w][t];
+                if (j <= i || !in_contact(a, b)) continue;
+                ++k;
+                if (want_candidate && first < 0) {
+                    // Weber number of the connection (foam_dynamics.rs:213-219).
+                    const float dx = b.x - a.x, dy = b.y - a.y, dz = b.z - a.z;
+                    const float dist = sqrtf(dx * dx + dy * dy + dz * dz);
+                    const float nx = dx / dist, ny = dy / dist, nz = dz / dist;
+                    const float4 va = vt[i < c.n ? i : c.n - 1], vb = vt[j];
+                    const float rel = (vb.x - va.x) * nx + (vb.y - va.y) * ny + (vb.z - va.z) * nz;
+                    const float weber = c.density * (rel * rel) * a.w / c.surface_tension;
+                    if (weber > c.coal_thr) first = static_cast<long long>(i) * c.n + j;
+                }
             }
+            wave_lds_fence();
         }
     }
     if (i >= c.n) return;
-    count[static_cast<size_t>(i) * c.nruns + run] = k;
-    if (want_candidate) cand[static_cast<size_t>(i) * c.nruns + run] = first;
+    count[static_cast<size_t>(run) * c.n + i] = k;
+    if (want_candidate) cand[static_cast<size_t>(run) * c.n + i] = first;
 }
 
-// Exclusive scan of count[m] into offs[m], total in offs[m]; first
-// coalescence candidate (smallest key >= 0, else -1) into cand_out.
-__global__ __launch_bounds__(1024) void cluster_scan_kernel(const int* __restrict__ count, size_t m,
-                                                            int* __restrict__ offs,
-                                                            const long long* __restrict__ cand,
-                                                            long long* __restrict__ cand_out) {
-    __shared__ int s_sum[1024];
-    __shared__ long long s_min[1024];
-    const int t = threadIdx.x;
-    const size_t per = (m + 1023) / 1024;
-    const size_t lo = std::min(m, t * per), hi = std::min(m, lo + per);
-    int local = 0;
-    long long best = -1;
-    for (size_t k = lo; k < hi; ++k) {
-        local += count[k];
-        if (cand) {
-            const long long x = cand[k];
-            if (x >= 0 && (best < 0 || x < best)) best = x;
+// What the host needs of a contact search.
+struct Contacts {
+    long long cand;      // smallest candidate key, -1 for none
+    long long total;     // connections
+};
+
+__device__ inline long long first_key(long long a, long long b) { return a < 0 ? b : b < 0 ? a : (b < a ? b : a); }
+
+// Exclusive offsets of count in (bubble, run) order, in two launches.  The
+// first: a block takes kTile bubbles, its waves kMaxRuns / 16 runs each, and
+// leaves offsets within the block, the block's total and its smallest
+// candidate.  Loads and stores are rows of 64 bubbles; one block walking the
+// whole array in (bubble, run) order took 437 us at n = 4096 where the two
+// take 8.2.
+constexpr int kMaxRuns = 64;
+constexpr int kScanWaves = 16;
+__global__ __launch_bounds__(64 * kScanWaves) void cluster_offsets_kernel(const int* __restrict__ count, Consts c,
+                                                                         const long long* __restrict__ cand,
+                                                                         int* __restrict__ offs,
+                                                                         Contacts* __restrict__ tiles) {
+    constexpr int R = kMaxRuns / kScanWaves;
+    __shared__ int s_sum[kScanWaves][kTile];
+    __shared__ long long s_cand[kScanWaves];
+    __shared__ int s_start[kTile];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int i = blockIdx.x * kTile + lane;
+    int v[R], sum = 0;
+    long long key = -1;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int run = w * R + r;
+        const bool in = i < c.n && run < c.nruns;
+        v[r] = in ? count[static_cast<size_t>(run) * c.n + i] : 0;
+        if (cand && in) key = first_key(key, cand[static_cast<size_t>(run) * c.n + i]);
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) sum += v[r];
+    s_sum[w][lane] = sum;
+    for (int d = 32; d > 0; d >>= 1) key = first_key(key, __shfl_xor(key, d));
+    if (lane == 0) s_cand[w] = key;
+    __syncthreads();
+    if (w == 0) {
+        int own = 0;
+        for (int k = 0; k < kScanWaves; ++k) own += s_sum[k][lane];
+        int incl = own;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int up = __shfl_up(incl, d);
+            if (lane >= d) incl += up;
+        }
+        s_start[lane] = incl - own;
+        if (lane == 63) {
+            for (int k = 0; k < kScanWaves; ++k) key = first_key(key, s_cand[k]);
+            tiles[blockIdx.x] = {key, incl};
         }
     }
-    s_sum[t] = local;
-    s_min[t] = best;
     __syncthreads();
-    for (int d = 1; d < 1024; d <<= 1) {
-        const int add = t >= d ? s_sum[t - d] : 0;
-        long long other = t >= d ? s_min[t - d] : -1;
+    int o = s_start[lane];
+    for (int k = 0; k < w; ++k) o += s_sum[k][lane];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int run = w * R + r;
+        if (i < c.n && run < c.nruns) offs[static_cast<size_t>(run) * c.n + i] = o;
+        o += v[r];
+    }
+}
+
+// The second: one block turns the tiles' totals into their first offsets and
+// leaves {smallest candidate, total} in *out.
+__global__ __launch_bounds__(1024) void cluster_tiles_kernel(Contacts* __restrict__ tiles, int ntiles,
+                                                             Contacts* __restrict__ out) {
+    __shared__ long long s_sum[16], s_key[16];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    long long base = 0, key = -1;
+    for (int b0 = 0; b0 < ntiles; b0 += 1024) {
+        const Contacts v = b0 + t < ntiles ? tiles[b0 + t] : Contacts{-1, 0};
+        key = first_key(key, v.cand);
+        long long incl = v.total;
+        for (int d = 1; d < 64; d <<= 1) {
+            const long long up = __shfl_up(incl, d);
+            if (lane >= d) incl += up;
+        }
+        if (lane == 63) s_sum[w] = incl;
         __syncthreads();
-        s_sum[t] += add;
-        if (other >= 0 && (s_min[t] < 0 || other < s_min[t])) s_min[t] = other;
+        long long before = base;
+        for (int k = 0; k < 16; ++k) {
+            if (k < w) before += s_sum[k];
+            base += s_sum[k];
+        }
+        if (b0 + t < ntiles) tiles[b0 + t].total = before + incl - v.total;
         __syncthreads();
     }
-    int run = s_sum[t] - local;    // exclusive prefix of this thread's chunk
-    for (size_t k = lo; k < hi; ++k) {
-        offs[k] = run;
-        run += count[k];
-    }
-    if (t == 1023) {
-        offs[m] = s_sum[1023];
-        if (cand_out) *cand_out = s_min[1023];
+    for (int d = 32; d > 0; d >>= 1) key = first_key(key, __shfl_xor(key, d));
+    if (lane == 0) s_key[w] = key;
+    __syncthreads();
+    if (t == 0) {
+        for (int k = 1; k < 16; ++k) key = first_key(key, s_key[k]);
+        *out = {key, base};
     }
 }
 
@@ -328,26 +423,31 @@ static_assert(sizeof(ConnRec) == sizeof(sf_cluster_connection), "connection reco
 __global__ __launch_bounds__(256) void cluster_connect_kernel(const float4* __restrict__ pr,
                                                               const float4* __restrict__ vt,
                                                               const uint32_t* __restrict__ ids, Consts c,
+                                                              const int* __restrict__ count,
                                                               const int* __restrict__ offs,
+                                                              const Contacts* __restrict__ tiles,
                                                               ConnRec* __restrict__ out) {
 #pragma clang fp contract(off)
     const int lane = threadIdx.x & 63;
-    const int run = blockIdx.y * kRunsPerBlock + (threadIdx.x >> 6);
+    const int run = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.y) * kRunsPerBlock +
+                                                   static_cast<int>(threadIdx.x >> 6));
     const int i = blockIdx.x * kTile + lane;
     if (run >= c.nruns) return;          // whole wave
+    int left = i < c.n ? count[static_cast<size_t>(run) * c.n + i] : 0;
+    if (__ballot(left > 0) == 0) return;
     const int ic = i < c.n ? i : c.n - 1;
     const float4 a = pr[ic];
     const float ta = vt[ic].w;
     const float pa = 4.0f * c.surface_tension / a.w;     // pressure_difference (foam.rs:72-74)
     const int j0 = run * c.run, j1 = min(c.n, j0 + c.run);
-    int k = i < c.n ? offs[static_cast<size_t>(i) * c.nruns + run] : 0;
-    for (int jc = j0; jc < j1; jc += 64) {
-        const float4 mine = pr[min(jc + lane, c.n - 1)];
-        const int cnt = min(64, j1 - jc);
-        for (int t = 0; t < cnt; ++t) {
-            const int j = jc + t;
-            const float4 b = lane_bcast(mine, t);
-            if (i >= c.n || j <= i || !in_contact(a, b)) continue;
+    size_t k = left > 0 ? static_cast<size_t>(tiles[blockIdx.x].total) + offs[static_cast<size_t>(run) * c.n + i] : 0;
+    for (int jc = j0; jc < j1; jc += kNear) {
+        unsigned mask = near_mask(pr + jc, a, min(kNear, j1 - jc), 1.3f, 1.f);
+        if (left == 0) mask = 0;
+        for (; mask; mask &= mask - 1) {
+            const int j = jc + __builtin_ctz(mask);
+            const float4 b = pr[j];
+            if (j <= i || !in_contact(a, b)) continue;
             // BubbleConnection::new (foam.rs:106-139).
             const float dx = b.x - a.x, dy = b.y - a.y, dz = b.z - a.z;
             const float dist = sqrtf(dx * dx + dy * dy + dz * dz);
@@ -405,8 +505,8 @@ struct Cluster {
     int* count = nullptr;
     int* offs = nullptr;
     long long* cand = nullptr;
-    long long* cand_out = nullptr;
-    size_t cnt_cap = 0;
+    Contacts* tiles = nullptr;      // per kTile bubbles, and the whole search's at the end
+    size_t cnt_cap = 0, tile_cap = 0;
     ConnRec* conn_dev = nullptr;
     size_t conn_cap = 0;
     // Host connection list and neighbour lists (valid when conn_valid).
@@ -434,7 +534,7 @@ struct Cluster {
             dfree(pr[k]);
             dfree(vt[k]);
         }
-        dfree(ids_dev); dfree(part); dfree(count); dfree(offs); dfree(cand); dfree(cand_out); dfree(conn_dev);
+        dfree(ids_dev); dfree(part); dfree(count); dfree(offs); dfree(cand); dfree(tiles); dfree(conn_dev);
         if (stream) (void)hipStreamDestroy(stream);
     }
 
@@ -467,7 +567,7 @@ struct Cluster {
     void reserve(int want) {
         if (want <= cap) return;
         const int nc = std::max(want, std::max(64, cap * 2));
-        float4* npr[2] = {dnew<float4>(nc), dnew<float4>(nc)};
+        float4* npr[2] = {dnew<float4>(nc + kNear), dnew<float4>(nc + kNear)};
         float4* nvt[2] = {dnew<float4>(nc), dnew<float4>(nc)};
         uint32_t* nid = dnew<uint32_t>(nc);
         if (n > 0) {
@@ -496,14 +596,24 @@ struct Cluster {
             part_cap = np;
         }
         const size_t m = static_cast<size_t>(c.nruns) * n;
-        if (m + 1 > cnt_cap) {
+        if (m > cnt_cap) {
             dfree(count); dfree(offs); dfree(cand);
-            count = dnew<int>(m + 1);
-            offs = dnew<int>(m + 1);
-            cand = dnew<long long>(m + 1);
-            cnt_cap = m + 1;
+            cnt_cap = 0;
+            count = offs = nullptr;
+            cand = nullptr;
+            count = dnew<int>(m);
+            offs = dnew<int>(m);
+            cand = dnew<long long>(m);
+            cnt_cap = m;
         }
-        if (!cand_out) cand_out = dnew<long long>(1);
+        const size_t nt = (n + kTile - 1) / kTile;
+        if (nt + 1 > tile_cap) {
+            dfree(tiles);
+            tiles = nullptr;
+            tile_cap = 0;
+            tiles = dnew<Contacts>(nt + 1);
+            tile_cap = nt + 1;
+        }
     }
 
     dim3 pair_grid(const Consts& c) const {
@@ -547,17 +657,17 @@ struct Cluster {
         hipLaunchKernelGGL(cluster_contact_kernel, pair_grid(c), dim3(256), 0, stream, pr[cur], vt[cur], c,
                            candidate ? 1 : 0, count, cand);
         SF_HIP(hipGetLastError());
-        const size_t m = static_cast<size_t>(c.nruns) * n;
-        hipLaunchKernelGGL(cluster_scan_kernel, dim3(1), dim3(1024), 0, stream, count, m, offs,
-                           candidate ? cand : nullptr, candidate ? cand_out : nullptr);
+        const int ntiles = (n + kTile - 1) / kTile;
+        hipLaunchKernelGGL(cluster_offsets_kernel, dim3(ntiles), dim3(64 * kScanWaves), 0, stream, count, c,
+                           candidate ? cand : nullptr, offs, tiles);
         SF_HIP(hipGetLastError());
-        int total = 0;
-        SF_HIP(hipMemcpyAsync(&total, offs + m, sizeof(int), hipMemcpyDeviceToHost, stream));
-        long long key = -1;
-        if (candidate) SF_HIP(hipMemcpyAsync(&key, cand_out, sizeof(long long), hipMemcpyDeviceToHost, stream));
+        hipLaunchKernelGGL(cluster_tiles_kernel, dim3(1), dim3(1024), 0, stream, tiles, ntiles, tiles + ntiles);
+        SF_HIP(hipGetLastError());
+        Contacts r;
+        SF_HIP(hipMemcpyAsync(&r, tiles + ntiles, sizeof(r), hipMemcpyDeviceToHost, stream));
         SF_HIP(hipStreamSynchronize(stream));
-        if (cand_key) *cand_key = key;
-        return total;
+        if (cand_key) *cand_key = r.cand;
+        return static_cast<int>(r.total);
     }
 
     // update_connections (foam.rs:321-360) on the current state, after
@@ -572,7 +682,7 @@ struct Cluster {
         conns.resize(total);
         if (total > 0) {
             hipLaunchKernelGGL(cluster_connect_kernel, pair_grid(c), dim3(256), 0, stream, pr[cur], vt[cur],
-                               ids_dev, c, offs, conn_dev);
+                               ids_dev, c, count, offs, tiles, conn_dev);
             SF_HIP(hipGetLastError());
             SF_HIP(hipMemcpyAsync(conns.data(), conn_dev, total * sizeof(ConnRec), hipMemcpyDeviceToHost, stream));
             SF_HIP(hipStreamSynchronize(stream));
