@@ -164,9 +164,83 @@ __global__ __launch_bounds__(64) void multi_diag_kernel(const double2* part, int
         hist[(slot0 + static_cast<int>(blockIdx.x)) % cap] = make_double2(m + fixed, l > 0.0 ? 2.0 / l : INFINITY);
 }
 
-__global__ void fill_kernel(float* p, size_t n, float v) {
+// Both halves of the ping-pong state from one value each.
+__global__ __launch_bounds__(256) void fill_kernel(float* h0, float* h1, float* l0, float* l1, float* g0, float* g1,
+                                                   size_t n, float h, float l, float g) {
     const size_t c = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x;
-    if (c < n) p[c] = v;
+    if (c >= n) return;
+    h0[c] = h1[c] = h;
+    l0[c] = l1[c] = l;
+    g0[c] = g1[c] = g;
+}
+
+// Exchange of fields with the host.  The host's FP64 arrays cross the link
+// once, as they are, and are split into both halves of the state (or joined
+// from it) here: splitting on the host and uploading each half took most of a
+// set_fields call (reset, set both fields, 48 steps, read both at 500 x 1003:
+// 1944 -> 1287 us, of which 950 are the link).  Bound by the link.
+//
+// Where cells [first, first + count) of a field come from: staged FP64, the
+// first half itself (just copied there; low word 0), or the current state.
+enum class From { kStage, kFirst, kState };
+
+template <From FROM>
+__global__ __launch_bounds__(256) void split_h_kernel(const double* stage, const float* src_hi, const float* src_lo,
+                                                      float* h0, float* h1, float* l0, float* l1, size_t count,
+                                                      float* part, bool first) {
+    float mx = 0.f;
+    for (size_t c = blockIdx.x * 256 + threadIdx.x; c < count; c += static_cast<size_t>(gridDim.x) * 256) {
+        float h, l = 0.f;
+        if (FROM == From::kStage) {
+            h = static_cast<float>(stage[c]);
+            l = static_cast<float>(stage[c] - static_cast<double>(h));
+        } else {
+            h = src_hi[c];
+            if (FROM == From::kState) l = src_lo[c];
+        }
+        h0[c] = h1[c] = h;
+        l0[c] = l1[c] = l;
+        mx = h > mx ? h : mx;          // a NaN is passed over
+    }
+    for (int d = 32; d > 0; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d));
+    __shared__ float s[4];
+    if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = mx;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        mx = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
+        part[blockIdx.x] = first ? mx : fmaxf(mx, part[blockIdx.x]);
+    }
+}
+
+template <From FROM>
+__global__ __launch_bounds__(256) void split_g_kernel(const double* stage, const float* src, float* g0, float* g1,
+                                                      size_t count) {
+    const size_t c = blockIdx.x * static_cast<size_t>(256) + threadIdx.x;
+    if (c < count) g0[c] = g1[c] = FROM == From::kStage ? static_cast<float>(stage[c]) : src[c];
+}
+
+template <class T>
+__global__ __launch_bounds__(256) void join_kernel(const float* hi, const float* lo, const float* g, size_t count,
+                                                   T* h_out, T* g_out) {
+    const size_t c = blockIdx.x * static_cast<size_t>(256) + threadIdx.x;
+    if (c >= count) return;
+    if (h_out) h_out[c] = static_cast<T>(static_cast<double>(hi[c]) + static_cast<double>(lo[c]));
+    if (g_out) g_out[c] = static_cast<T>(g[c]);
+}
+
+// out: both pole rows' high words, their low words, and the largest of part.
+__global__ __launch_bounds__(256) void pole_rows_kernel(const float* hi, const float* lo, int nt, int np,
+                                                        const float* part, int nparts, float* out) {
+    const size_t last = static_cast<size_t>(nt - 1) * np;
+    for (int c = blockIdx.x * 256 + threadIdx.x; c < 4 * np; c += gridDim.x * 256) {
+        const int row = c / np, j = c - row * np;
+        out[c] = (row < 2 ? hi : lo)[(row & 1 ? last : 0) + j];
+    }
+    if (blockIdx.x != 0 || threadIdx.x >= 64) return;
+    float mx = 0.f;
+    for (int k = threadIdx.x; k < nparts; k += 64) mx = fmaxf(mx, part[k]);
+    for (int d = 32; d > 0; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d));
+    if (threadIdx.x == 0) out[4 * static_cast<size_t>(np)] = mx;
 }
 
 // ---------------------------------------------------------------------------
@@ -338,6 +412,8 @@ Drainage::Drainage(const sf_params& prm, int n_theta, int n_phi) : p(prm), nt(n_
     diag_hist = dalloc<double2>(kHistCap);
     stats_part = dalloc<StatsPart>(kStatsBlocks);
     stats_out = dalloc<StatsPart>(1);
+    split_part = dalloc<float>(kSplitBlocks);
+    pole_rows = dalloc<float>(4 * static_cast<size_t>(np) + 1);
     tables_dirty = true;
 }
 
@@ -350,6 +426,7 @@ Drainage::~Drainage() {
     for (int k = 0; k < kDiagBufs; ++k) dfree(diag_part[k]);
     dfree(multi_part); dfree(lo_mid); dfree(hpole_mid[0]); dfree(hpole_mid[1]);
     dfree(stats_part); dfree(stats_out); dfree(gather_idx); dfree(gather_out);
+    dfree(split_part); dfree(pole_rows); dfree(stage);
     dfree(rgb); dfree(cmf_dev); dfree(spec_rows); dfree(spec_cols); dfree(spec_view); dfree(caustic);
     step_timer.destroy();
     spec_timer.destroy();
@@ -413,66 +490,105 @@ void Drainage::upload_tables() {
 }
 
 // FP64 pole-row film volume, used while the h poles are copied through.
-void Drainage::update_fixed_pole_mass() {
-    std::vector<float> h0(2 * static_cast<size_t>(np)), l0(2 * static_cast<size_t>(np));
-    SF_HIP(hipMemcpyAsync(h0.data(), hi[cur_hi], np * sizeof(float), hipMemcpyDeviceToHost, stream));
-    SF_HIP(hipMemcpyAsync(l0.data(), lo[cur], np * sizeof(float), hipMemcpyDeviceToHost, stream));
-    SF_HIP(hipMemcpyAsync(h0.data() + np, hi[cur_hi] + (nt - 1) * static_cast<size_t>(np),
-                          np * sizeof(float), hipMemcpyDeviceToHost, stream));
-    SF_HIP(hipMemcpyAsync(l0.data() + np, lo[cur] + (nt - 1) * static_cast<size_t>(np),
-                          np * sizeof(float), hipMemcpyDeviceToHost, stream));
+// The pole rows' film volume, added up on the host in column order, and the
+// largest thickness where the last split left its maxima.
+void Drainage::update_fixed_pole_mass(bool with_max) {
+    const size_t w = static_cast<size_t>(np);
+    hipLaunchKernelGGL(pole_rows_kernel, dim3(std::min<unsigned>(cdiv(4 * w, 256), 256)), dim3(256), 0, stream,
+                       hi[cur_hi], lo[cur], nt, np, split_part, with_max ? kSplitBlocks : 0, pole_rows);
+    SF_HIP(hipGetLastError());
+    std::vector<float> r(4 * w + 1);
+    SF_HIP(hipMemcpyAsync(r.data(), pole_rows, r.size() * sizeof(float), hipMemcpyDeviceToHost, stream));
     SF_HIP(hipStreamSynchronize(stream));
     double st = 0.0, sb = 0.0;
-    for (int j = 0; j < np; ++j) {
-        st += static_cast<double>(h0[j]) + static_cast<double>(l0[j]);
-        sb += static_cast<double>(h0[np + j]) + static_cast<double>(l0[np + j]);
+    for (size_t j = 0; j < w; ++j) {
+        st += static_cast<double>(r[j]) + static_cast<double>(r[2 * w + j]);
+        sb += static_cast<double>(r[w + j]) + static_cast<double>(r[3 * w + j]);
     }
     pole_mass_fixed = pole_area_top * st + pole_area_bot * sb;
+    if (with_max) h_max = r[4 * w];
 }
 
-// Uploads hi/lo/Γ into both ping-pong halves so that rows a step never
-// writes (the poles, and Γ when it is frozen) hold the same values in both.
-void Drainage::upload(const float* h_hi, const float* h_lo, const float* gam) {
-    if (h_hi) {
-        // independent maxima, so that the loop vectorises
-        float mx[32] = {0.f};
-        size_t k0 = 0;
-        for (; k0 + 32 <= n; k0 += 32)
-            for (int j = 0; j < 32; ++j) mx[j] = h_hi[k0 + j] > mx[j] ? h_hi[k0 + j] : mx[j];
-        for (; k0 < n; ++k0) mx[0] = std::max(mx[0], h_hi[k0]);
-        h_max = *std::max_element(mx, mx + 32);
-        for (int k = 0; k < 2; ++k) {
-            SF_HIP(hipMemcpyAsync(hi[k], h_hi, n * sizeof(float), hipMemcpyHostToDevice, stream));
-            SF_HIP(hipMemcpyAsync(lo[k], h_lo, n * sizeof(float), hipMemcpyHostToDevice, stream));
+// Two fields' worth of kStageCells FP64 cells, at most.
+double* Drainage::ensure_stage() {
+    if (!stage) stage = dalloc<double>(2 * std::min(n, kStageCells));
+    return stage;
+}
+
+// Sets the fields from host arrays (nullptr: keeps one), in both ping-pong
+// halves so that rows a step never writes (the poles, and Γ when it is
+// frozen) hold the same values in both.
+template <class T>
+void Drainage::upload(const T* h, const T* gam) {
+    constexpr bool wide = sizeof(T) == 8;
+    double* const st = wide && (h || gam) ? ensure_stage() : nullptr;
+    const size_t chunk = wide ? std::min(n, kStageCells) : n;
+    if (!h) {
+        hipLaunchKernelGGL(split_h_kernel<From::kState>, dim3(kSplitBlocks), dim3(256), 0, stream, nullptr, hi[cur_hi],
+                           lo[cur], hi[0], hi[1], lo[0], lo[1], n, split_part, true);
+        SF_HIP(hipGetLastError());
+    }
+    if (!gam) {
+        hipLaunchKernelGGL(split_g_kernel<From::kState>, dim3(cdiv(n, 256)), dim3(256), 0, stream, nullptr, g[cur_g],
+                           g[0], g[1], n);
+        SF_HIP(hipGetLastError());
+    }
+    for (size_t c = 0; c < n; c += chunk) {
+        const size_t m = std::min(chunk, n - c);
+        if (h) {
+            SF_HIP(hipMemcpyAsync(wide ? static_cast<void*>(st) : hi[0], h + c, m * sizeof(T), hipMemcpyHostToDevice,
+                                  stream));
+            hipLaunchKernelGGL(split_h_kernel<(wide ? From::kStage : From::kFirst)>, dim3(kSplitBlocks), dim3(256), 0,
+                               stream, st, hi[0] + c, nullptr, hi[0] + c, hi[1] + c, lo[0] + c, lo[1] + c, m,
+                               split_part, c == 0);
+            SF_HIP(hipGetLastError());
+        }
+        if (gam) {
+            double* const sg = wide ? st + chunk : nullptr;
+            SF_HIP(hipMemcpyAsync(wide ? static_cast<void*>(sg) : g[0], gam + c, m * sizeof(T), hipMemcpyHostToDevice,
+                                  stream));
+            hipLaunchKernelGGL(split_g_kernel<(wide ? From::kStage : From::kFirst)>, dim3(cdiv(m, 256)), dim3(256), 0,
+                               stream, sg, g[0] + c, g[0] + c, g[1] + c, m);
+            SF_HIP(hipGetLastError());
         }
     }
-    if (gam) {
-        for (int k = 0; k < 2; ++k)
-            SF_HIP(hipMemcpyAsync(g[k], gam, n * sizeof(float), hipMemcpyHostToDevice, stream));
-    }
-    SF_HIP(hipStreamSynchronize(stream));
     cur = cur_hi = cur_g = 0;
     since_rebase = 0;
     poles_virtual = false;
-    update_fixed_pole_mass();
+    update_fixed_pole_mass(true);
+}
+
+// The current fields into host arrays (nullptr: not wanted).
+template <class T>
+void Drainage::download(T* h, T* gam) {
+    T* const st = reinterpret_cast<T*>(ensure_stage());
+    const size_t chunk = std::min(n, kStageCells);
+    for (size_t c = 0; c < n; c += chunk) {
+        const size_t m = std::min(chunk, n - c);
+        hipLaunchKernelGGL(join_kernel<T>, dim3(cdiv(m, 256)), dim3(256), 0, stream, hi[cur_hi] + c, lo[cur] + c,
+                           g[cur_g] + c, m, h ? st : nullptr, gam ? st + chunk : nullptr);
+        SF_HIP(hipGetLastError());
+        if (h) SF_HIP(hipMemcpyAsync(h + c, st, m * sizeof(T), hipMemcpyDeviceToHost, stream));
+        if (gam) SF_HIP(hipMemcpyAsync(gam + c, st + chunk, m * sizeof(T), hipMemcpyDeviceToHost, stream));
+    }
+    SF_HIP(hipStreamSynchronize(stream));
 }
 
 void Drainage::fill(double h0, double gamma0) {
     const float h_hi = static_cast<float>(h0);
     const float h_lo = static_cast<float>(h0 - static_cast<double>(h_hi));
     h_max = h0;
-    for (int k = 0; k < 2; ++k) {
-        hipLaunchKernelGGL(fill_kernel, dim3(cdiv(n, 256)), dim3(256), 0, stream, hi[k], n, h_hi);
-        hipLaunchKernelGGL(fill_kernel, dim3(cdiv(n, 256)), dim3(256), 0, stream, lo[k], n, h_lo);
-        hipLaunchKernelGGL(fill_kernel, dim3(cdiv(n, 256)), dim3(256), 0, stream, g[k], n,
-                           static_cast<float>(gamma0));
-    }
+    hipLaunchKernelGGL(fill_kernel, dim3(cdiv(n, 256)), dim3(256), 0, stream, hi[0], hi[1], lo[0], lo[1], g[0], g[1], n,
+                       h_hi, h_lo, static_cast<float>(gamma0));
     SF_HIP(hipGetLastError());
     SF_HIP(hipStreamSynchronize(stream));
     cur = cur_hi = cur_g = 0;
     since_rebase = 0;
     poles_virtual = false;
-    update_fixed_pole_mass();
+    // as update_fixed_pole_mass adds rows of this value
+    double row = 0.0;
+    for (int j = 0; j < np; ++j) row += static_cast<double>(h_hi) + static_cast<double>(h_lo);
+    pole_mass_fixed = pole_area_top * row + pole_area_bot * row;
 }
 
 // ---------------------------------------------------------------------------
@@ -1099,56 +1215,16 @@ extern "C" int sf_drainage_get_params(const sf_drainage* ctx, sf_params* out) {
 extern "C" int sf_drainage_set_fields(sf_drainage* ctx, const float* h, const float* gamma) {
     return guard([&] {
         SF_REQUIRE(ctx != nullptr, SF_ERR_INVALID, "ctx is NULL");
-        Drainage* d = D(ctx);
-        d->materialize();
-        std::vector<float> zeros;
-        if (h) zeros.assign(d->n, 0.f);
-        if (!h) {
-            // keep h: copy the current one into both halves
-            std::vector<float> hh(d->n), ll(d->n);
-            SF_HIP(hipMemcpyAsync(hh.data(), d->hi[d->cur_hi], d->n * 4, hipMemcpyDeviceToHost, d->stream));
-            SF_HIP(hipMemcpyAsync(ll.data(), d->lo[d->cur], d->n * 4, hipMemcpyDeviceToHost, d->stream));
-            SF_HIP(hipStreamSynchronize(d->stream));
-            if (!gamma) {
-                std::vector<float> gg(d->n);
-                SF_HIP(hipMemcpy(gg.data(), d->g[d->cur_g], d->n * 4, hipMemcpyDeviceToHost));
-                d->upload(hh.data(), ll.data(), gg.data());
-            } else {
-                d->upload(hh.data(), ll.data(), gamma);
-            }
-            return;
-        }
-        if (!gamma) {
-            std::vector<float> gg(d->n);
-            SF_HIP(hipMemcpy(gg.data(), d->g[d->cur_g], d->n * 4, hipMemcpyDeviceToHost));
-            d->upload(h, zeros.data(), gg.data());
-        } else {
-            d->upload(h, zeros.data(), gamma);
-        }
+        D(ctx)->materialize();
+        D(ctx)->upload(h, gamma);
     });
 }
 
 extern "C" int sf_drainage_set_fields_f64(sf_drainage* ctx, const double* h, const double* gamma) {
     return guard([&] {
         SF_REQUIRE(ctx != nullptr, SF_ERR_INVALID, "ctx is NULL");
-        Drainage* d = D(ctx);
-        d->materialize();
-        std::vector<float> hh(d->n), ll(d->n), gg(d->n);
-        if (h) {
-            for (size_t k = 0; k < d->n; ++k) {
-                hh[k] = static_cast<float>(h[k]);
-                ll[k] = static_cast<float>(h[k] - static_cast<double>(hh[k]));
-            }
-        } else {
-            SF_HIP(hipMemcpy(hh.data(), d->hi[d->cur_hi], d->n * 4, hipMemcpyDeviceToHost));
-            SF_HIP(hipMemcpy(ll.data(), d->lo[d->cur], d->n * 4, hipMemcpyDeviceToHost));
-        }
-        if (gamma) {
-            for (size_t k = 0; k < d->n; ++k) gg[k] = static_cast<float>(gamma[k]);
-        } else {
-            SF_HIP(hipMemcpy(gg.data(), d->g[d->cur_g], d->n * 4, hipMemcpyDeviceToHost));
-        }
-        d->upload(hh.data(), ll.data(), gg.data());
+        D(ctx)->materialize();
+        D(ctx)->upload(h, gamma);
     });
 }
 
@@ -1165,38 +1241,16 @@ extern "C" int sf_drainage_step(sf_drainage* ctx, int32_t n_steps, double dt) {
 extern "C" int sf_drainage_copy_field(sf_drainage* ctx, float* h, float* gamma) {
     return guard([&] {
         SF_REQUIRE(ctx != nullptr, SF_ERR_INVALID, "ctx is NULL");
-        Drainage* d = D(ctx);
-        d->materialize();
-        if (h) {
-            std::vector<float> ll(d->n);
-            SF_HIP(hipMemcpyAsync(h, d->hi[d->cur_hi], d->n * 4, hipMemcpyDeviceToHost, d->stream));
-            SF_HIP(hipMemcpyAsync(ll.data(), d->lo[d->cur], d->n * 4, hipMemcpyDeviceToHost, d->stream));
-            SF_HIP(hipStreamSynchronize(d->stream));
-            for (size_t k = 0; k < d->n; ++k)
-                h[k] = static_cast<float>(static_cast<double>(h[k]) + static_cast<double>(ll[k]));
-        }
-        if (gamma) {
-            SF_HIP(hipMemcpyAsync(gamma, d->g[d->cur_g], d->n * 4, hipMemcpyDeviceToHost, d->stream));
-            SF_HIP(hipStreamSynchronize(d->stream));
-        }
+        D(ctx)->materialize();
+        D(ctx)->download(h, gamma);
     });
 }
 
 extern "C" int sf_drainage_copy_field_f64(sf_drainage* ctx, double* h, double* gamma) {
     return guard([&] {
         SF_REQUIRE(ctx != nullptr, SF_ERR_INVALID, "ctx is NULL");
-        Drainage* d = D(ctx);
-        d->materialize();
-        std::vector<float> hh(d->n), ll(d->n), gg(d->n);
-        SF_HIP(hipMemcpyAsync(hh.data(), d->hi[d->cur_hi], d->n * 4, hipMemcpyDeviceToHost, d->stream));
-        SF_HIP(hipMemcpyAsync(ll.data(), d->lo[d->cur], d->n * 4, hipMemcpyDeviceToHost, d->stream));
-        SF_HIP(hipMemcpyAsync(gg.data(), d->g[d->cur_g], d->n * 4, hipMemcpyDeviceToHost, d->stream));
-        SF_HIP(hipStreamSynchronize(d->stream));
-        if (h)
-            for (size_t k = 0; k < d->n; ++k)
-                h[k] = static_cast<double>(hh[k]) + static_cast<double>(ll[k]);
-        if (gamma)
-            for (size_t k = 0; k < d->n; ++k) gamma[k] = static_cast<double>(gg[k]);
+        D(ctx)->materialize();
+        D(ctx)->download(h, gamma);
     });
 }
 
@@ -1350,15 +1404,20 @@ extern "C" int sf_drainage_history(sf_drainage* ctx, int32_t n, double* mass, do
         d->finalize_diag();
         const int64_t avail = std::min<int64_t>(d->hist_count, Drainage::kHistCap);
         const int64_t m = std::min<int64_t>(avail, n);
-        std::vector<double2> all(Drainage::kHistCap);
-        SF_HIP(hipMemcpyAsync(all.data(), d->diag_hist, Drainage::kHistCap * sizeof(double2),
-                              hipMemcpyDeviceToHost, d->stream));
+        // the last m entries of the ring, oldest first: up to two runs
+        std::vector<double2> last(static_cast<size_t>(m));
+        const int64_t from = (d->hist_count - m) % Drainage::kHistCap;
+        const int64_t run = std::min<int64_t>(m, Drainage::kHistCap - from);
+        if (run > 0)
+            SF_HIP(hipMemcpyAsync(last.data(), d->diag_hist + from, run * sizeof(double2), hipMemcpyDeviceToHost,
+                                  d->stream));
+        if (m > run)
+            SF_HIP(hipMemcpyAsync(last.data() + run, d->diag_hist, (m - run) * sizeof(double2), hipMemcpyDeviceToHost,
+                                  d->stream));
         SF_HIP(hipStreamSynchronize(d->stream));
         for (int64_t k = 0; k < m; ++k) {
-            const int64_t step = d->hist_count - m + k;
-            const double2 e = all[static_cast<size_t>(step % Drainage::kHistCap)];
-            if (mass) mass[k] = e.x;
-            if (dt_cfl) dt_cfl[k] = e.y;
+            if (mass) mass[k] = last[k].x;
+            if (dt_cfl) dt_cfl[k] = last[k].y;
         }
         if (n_out) *n_out = static_cast<int32_t>(m);
     });

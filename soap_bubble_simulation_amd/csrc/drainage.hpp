@@ -70,6 +70,13 @@ struct Drainage {
     // per block and the most steps, 0 where it is not used.
     int multi_rows = 1, multi_steps = 0;
     double2* multi_part = nullptr;
+    // Field exchange with the host: FP64 staging (at most 2 kStageCells
+    // cells, made at the first use), maxima per block, pole rows.
+    static constexpr size_t kStageCells = size_t{1} << 21;
+    static constexpr int kSplitBlocks = 512;
+    double* stage = nullptr;
+    float* split_part = nullptr;
+    float* pole_rows = nullptr;
 
     // device state (see drainage_kernels.hpp for the layout)
     float* hi[2] = {nullptr, nullptr};
@@ -161,8 +168,12 @@ struct Drainage {
     Drainage& operator=(const Drainage&) = delete;
 
     void upload_tables();
-    void update_fixed_pole_mass();
-    void upload(const float* h_hi, const float* h_lo, const float* gam);
+    void update_fixed_pole_mass(bool with_max = false);
+    template <class T>
+    void upload(const T* h, const T* gam);
+    template <class T>
+    void download(T* h, T* gam);
+    double* ensure_stage();
     void fill(double h0, double gamma0);
     void front_columns(HostFront& f) const;
     void spawn_front();
