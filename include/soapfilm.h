@@ -410,7 +410,11 @@ int sf_foam_use_graph(sf_foam* foam, int32_t enable);
  * starts at an odd step of the 8-step renormalisation cycle, takes one step
  * per launch where needed.  In foams where two steps are possible a column
  * chunk holds 62 lanes' columns in both modes (lanes 0 and 63 form the
- * two-step kernel's halo columns), so both give identical results.  No counterpart
+ * two-step kernel's halo columns), so both give identical results.  Small
+ * foams (rows of at most 1024 columns, up to 2 blocks of at most 16 rows per
+ * compute unit) take up to 8 steps per launch by themselves, with pole means
+ * from FP64 ring sums; a call here, or explicit tile shapes, switches that
+ * off.  No counterpart
  * in the reference (foam.rs keeps no per-bubble grids). */
 int sf_foam_set_steps_per_launch(sf_foam* foam, int32_t steps);
 int sf_foam_get_steps_per_launch(sf_foam* foam, int32_t* steps);

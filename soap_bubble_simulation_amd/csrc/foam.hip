@@ -628,6 +628,150 @@ __global__ __launch_bounds__(256) void foam_step2_kernel(const FoamArgs a, const
     else foam_band2<4, false, REBASE>(a, it, B, lane, ring[wave]);
 }
 
+// ---- several steps per launch of a small foam -------------------------------
+//
+// A launch of one step costs a small foam 4.2-4.6 us, nearly all latency (24
+// bubbles of 16-64 latitudes: 0.3 us of traffic).  As drainage_multi_kernel
+// does for one film, a block owns whole rows [r0, r1) of one bubble, holds
+// them and `steps` halo rows a side in LDS and advances them `steps` times,
+// one row less a side each time, forming the ring means itself.  Cells are
+// foam_cell's; ring sums are FP64, in column order over fixed threads, and
+// pass between launches as float pairs, so that a run does not depend on how
+// it is cut into launches.  Bound by the latency of a step: 4.0 -> 2.6 us per step
+// there.
+constexpr int kFoamMultiSteps = 8;
+constexpr int kFoamMultiThreads = 1024;
+constexpr int kFoamMultiCells = 8;      // cells a thread updates per step, at most
+constexpr int kFoamMultiCols = kFoamMultiThreads;   // longest row: a ring column per thread
+constexpr int kFoamMultiBlocks = 2;   // blocks per CU, at most
+constexpr int kFoamMultiRows = 16;      // rows a block owns, at most
+constexpr size_t kFoamMultiLds = 150 * 1024;
+
+struct FoamMultiItem {
+    int bubble, r0, r1, pad;
+};
+
+template <bool REBASE>
+__global__ __launch_bounds__(kFoamMultiThreads) void foam_multi_kernel(const FoamArgs a, const FoamMultiItem* items,
+                                                                       int steps, int rebase_step) {
+    constexpr int T = kFoamMultiThreads, kWaves = T / 64;
+    extern __shared__ __align__(16) float lds_state[];
+    __shared__ float4 s_row[kFoamMultiRows + 2 * kFoamMultiSteps];
+    __shared__ double s_ring[2][kWaves];
+    const FoamMultiItem it = items[blockIdx.x];
+    const FoamBubble B = a.bub[it.bubble];
+    const int np = B.np, nt = B.nt, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int r0 = it.r0, r1 = it.r1;
+    const int e0 = max(r0 - steps, 0), e1 = min(r1 + steps, nt);
+    const int cells = (e1 - e0) * np;
+    float2* HL = reinterpret_cast<float2*>(lds_state);       // (hi, lo) of the block's rows
+    float* G = lds_state + 2 * cells;
+    {
+        const int64_t base = B.off + static_cast<int64_t>(e0) * np;
+        for (int c = tid; c < cells; c += T) {
+            HL[c] = make_float2(a.hi_in[base + c], a.lo_in[base + c]);
+            G[c] = a.g_in[base + c];
+        }
+    }
+    if (tid < e1 - e0) {
+        const FoamRow rl = a.rows[B.row_off + e0 + tid];
+        s_row[tid] = make_float4(rl.G1, rl.G2, B.dtc * rl.sin_t, 0.f);
+    }
+    float2 mean[2] = {make_float2(0.f, 0.f), make_float2(0.f, 0.f)}, total[2] = {mean[0], mean[0]};
+    bool have = a.pole_mean != 0;
+    if (have && e0 == 0) mean[0] = pole_mean(a.hpole_in + B.pole_off, B.nchunks, B.np_f);
+    if (have && e1 == nt) mean[1] = pole_mean(a.hpole_in + B.pole_off + B.nchunks, B.nchunks, B.np_f);
+    // A thread's cells lie T apart in the step's rows; row and column of each
+    // relative to the first row are the same in every step.
+    int rel[kFoamMultiCells], col[kFoamMultiCells];
+    rel[0] = tid / np;
+    col[0] = tid - rel[0] * np;
+    const int dr = T / np, dc = T - dr * np;
+#pragma unroll
+    for (int q = 1; q < kFoamMultiCells; ++q) {
+        rel[q] = rel[q - 1] + dr;
+        col[q] = col[q - 1] + dc;
+        if (col[q] >= np) {
+            col[q] -= np;
+            ++rel[q];
+        }
+    }
+    __syncthreads();
+    for (int k = 0; k < steps; ++k) {
+        const int left = steps - 1 - k;
+        const int u0 = max(1, r0 - left), u1 = min(nt - 1, r1 + left);      // rows updated in this step
+        const int count = (u1 - u0) * np, first = (u0 - e0) * np;
+        const bool rebase = REBASE && k == rebase_step;
+        const bool top = u0 == 1, bottom = u1 == nt - 1;
+        float2 nhl[kFoamMultiCells];
+        float ng[kFoamMultiCells];
+#pragma unroll
+        for (int q = 0; q < kFoamMultiCells; ++q) {
+            if (q * T >= count) break;                                      // uniform
+            const bool in = tid + q * T < count;
+            // out of range: the first cell again, not stored
+            const int c = in ? first + tid + q * T : first, i = in ? u0 + rel[q] : u0, j = in ? col[q] : 0;
+            const int w = j == 0 ? c + np - 1 : c - 1, e = j + 1 == np ? c - np + 1 : c + 1;
+            const float4 rw = s_row[i - e0];
+            const float2 C = HL[c], Wv = HL[w], Ev = HL[e];
+            float2 N = HL[c - np], S = HL[c + np];
+            if (have && i == 1) N = mean[0];
+            if (have && i == nt - 2) S = mean[1];
+            float lo_new, g_new;
+            foam_cell(B, rw.x, rw.y, rw.z, C.x, C.y, G[c], N.x, N.y, G[c - np], S.x, S.y, G[c + np], Wv.x, Wv.y, G[w],
+                      Ev.x, Ev.y, G[e], lo_new, g_new);
+            nhl[q] = make_float2(C.x, lo_new);
+            if (rebase) two_sum(C.x, lo_new, nhl[q].x, nhl[q].y);
+            ng[q] = g_new;
+        }
+        __syncthreads();                         // every neighbour is read
+#pragma unroll
+        for (int q = 0; q < kFoamMultiCells; ++q) {
+            if (q * T >= count) break;
+            if (tid + q * T < count) {
+                HL[first + tid + q * T] = nhl[q];
+                G[first + tid + q * T] = ng[q];
+            }
+        }
+        __syncthreads();                         // the new rows are written
+        if (top || bottom) {                     // uniform
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                if (!(e == 0 ? top : bottom)) continue;
+                const float2 v = tid < np ? HL[((e == 0 ? 1 : nt - 2) - e0) * np + tid] : make_float2(0.f, 0.f);
+                const double r = wave_sum(static_cast<double>(v.x) + static_cast<double>(v.y));
+                if (lane == 0) s_ring[e][wave] = r;
+            }
+            __syncthreads();
+            // every wave folds the waves' sums; written again only past the
+            // next step's first barrier
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                if (!(e == 0 ? top : bottom)) continue;
+                total[e] = split_pair(sf::lane_value(row_sum(lane < kWaves ? s_ring[e][lane] : 0.0), kWaves - 1));
+                mean[e] = pole_mean_of_sum(total[e], B.np_f);
+            }
+        }
+        have = true;
+    }
+    {
+        const int from = (r0 - e0) * np, own = (r1 - r0) * np;
+        const int64_t base = B.off + static_cast<int64_t>(r0) * np;
+        for (int c = tid; c < own; c += T) {
+            const float2 v = HL[from + c];
+            if (REBASE) a.hi_out[base + c] = v.x;
+            a.lo_out[base + c] = v.y;
+            a.g_out[base + c] = G[from + c];
+        }
+    }
+    // Ring sums for the next launch: the total in the first chunk's place.
+    for (int e = 0; e < 2; ++e) {
+        if (e == 0 ? r0 != 1 : r1 != nt - 1) continue;
+        for (int t = tid; t < B.nchunks; t += T)
+            a.hpole_out[B.pole_off + e * B.nchunks + t] = t == 0 ? total[e] : make_float2(0.f, 0.f);
+    }
+}
+
 // Writes every bubble's pole rows from the ring partials (one block per bubble).
 __global__ void foam_poles_kernel(float* hi, float* lo, const float2* hpole, const FoamBubble* bub) {
     const FoamBubble B = bub[blockIdx.x];
@@ -737,6 +881,13 @@ struct Foam {
     // this foam (every bubble at least 4 x 8).
     int steps_per_launch = 2;
     bool two_ok = false;
+    // Several steps per launch (foam_multi_kernel): the most steps (0: not
+    // used), blocks, bytes of LDS a block.
+    bool multi_allowed = true;
+    int multi_steps = 0, multi_blocks = 0;
+    size_t multi_lds = 0;
+    FoamMultiItem* d_multi = nullptr;
+    int multi_cap = 0;
     float2* hpole[2] = {nullptr, nullptr};
     int pole_slots = 0;
     FoamRow* rows = nullptr;
@@ -766,6 +917,7 @@ struct Foam {
         for (int k = 0; k < 2; ++k) {
             (void)hipFree(hi[k]); (void)hipFree(lo[k]); (void)hipFree(g[k]); (void)hipFree(hpole[k]);
         }
+        (void)hipFree(d_multi);
         (void)hipFree(rows); (void)hipFree(d_bub); (void)hipFree(d_items); (void)hipFree(d_area);
         (void)hipFree(d_lamg); (void)hipFree(d_sinab); (void)hipFree(d_coef3); (void)hipFree(d_stat);
         timer.destroy();
@@ -799,6 +951,98 @@ struct Foam {
             const int r0 = 1 + static_cast<int>(static_cast<int64_t>(rows) * k / nbands);
             const int r1 = 1 + static_cast<int>(static_cast<int64_t>(rows) * (k + 1) / nbands);
             for (int ch = 0; ch < B.nchunks; ++ch) items.push_back(FoamItem{b, r0, r1, ch * B.cw, ch, {0, 0, 0}});
+        }
+    }
+
+    // Rows a block of foam_multi_kernel owns of bubble b where a step of a
+    // block is to update at most `cells` cells.
+    static int multi_rows(const FoamBubble& B, int k, int cells) {
+        return std::max(1, std::min({cells / B.np - (k - 1), kFoamMultiRows, B.nt - 2}));
+    }
+
+    // Blocks of foam_multi_kernel for the foam's active bubbles: the least
+    // cells a block and step that keep one block per CU (two where one does
+    // not fit), so that wide and narrow bubbles' blocks take alike;
+    // sqrt(10^4 / n_phi) steps of the widest bubble, as Drainage::multi_plan.
+    // us per step, one-step launches -> these: 6 bubbles of 16-24 latitudes
+    // 3.9 -> 1.9, 100 of 24-48 5.3 -> 2.8, 16 of 64-256 8.0 -> 5.2; two blocks
+    // per CU: 200 of 16-40 5.8 -> 4.9, 30 of 64-256 10.6 -> 8.8.  At three and
+    // four, 300 of 16-32 lost (5.6 -> 7.1): those foams keep the streaming
+    // kernels.
+    void multi_plan() {
+        multi_steps = 0;
+        int np = 0;
+        for (int b = 0; b < nb; ++b)
+            if (active[b]) np = std::max(np, bub[b].np);
+        if (!multi_allowed || np == 0 || np > kFoamMultiCols) return;
+        const int k = std::max(2, std::min(static_cast<int>(std::lround(std::sqrt(1e4 / np))), kFoamMultiSteps));
+        auto blocks = [&](int cells) {
+            int64_t n = 0;
+            for (int b = 0; b < nb; ++b)
+                if (active[b]) n += (bub[b].nt - 2 + multi_rows(bub[b], k, cells) - 1) / multi_rows(bub[b], k, cells);
+            return n;
+        };
+        constexpr int kMost = kFoamMultiCells * kFoamMultiThreads;
+        int most = n_cu;
+        while (most <= kFoamMultiBlocks * n_cu && blocks(kMost) > most) most += n_cu;
+        if (most > kFoamMultiBlocks * n_cu) return;
+        int lo = 0, hi_ = kMost;                   // least cells that fit, by bisection
+        while (hi_ - lo > 1) {
+            const int mid = (lo + hi_) / 2;
+            (blocks(mid) <= most ? hi_ : lo) = mid;
+        }
+        std::vector<FoamMultiItem> items;
+        size_t held = 0, updated = 0;
+        for (int b = 0; b < nb; ++b) {
+            if (!active[b]) continue;
+            const FoamBubble& B = bub[b];
+            const int r = multi_rows(B, k, hi_);
+            for (int r0 = 1; r0 < B.nt - 1; r0 += r) items.push_back({b, r0, std::min(r0 + r, B.nt - 1), 0});
+            held = std::max(held, static_cast<size_t>(r + 2 * k) * B.np);
+            updated = std::max(updated, static_cast<size_t>(r + 2 * (k - 1)) * B.np);
+        }
+        if (items.empty() || held * 12 > kFoamMultiLds || updated > static_cast<size_t>(kMost)) return;
+        if (static_cast<int>(items.size()) > multi_cap) {
+            (void)hipFree(d_multi);
+            d_multi = nullptr;
+            multi_cap = 0;
+            d_multi = falloc<FoamMultiItem>(items.size());
+            multi_cap = static_cast<int>(items.size());
+        }
+        SF_HIP(hipMemcpyAsync(d_multi, items.data(), items.size() * sizeof(FoamMultiItem), hipMemcpyHostToDevice,
+                              stream));
+        SF_HIP(hipStreamSynchronize(stream));
+        for (const void* fn : {reinterpret_cast<const void*>(&foam_multi_kernel<false>),
+                               reinterpret_cast<const void*>(&foam_multi_kernel<true>)})
+            SF_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kFoamMultiLds)));
+        multi_steps = k;
+        multi_blocks = static_cast<int>(items.size());
+        multi_lds = held * 12;
+    }
+
+    // k steps in one launch of foam_multi_kernel (1 <= k <= multi_steps).
+    void step_multi(int k) {
+        const int to_rebase = 7 - since_rebase;            // the step after which hi, lo are renormalised
+        const bool rebase = to_rebase < k;
+        const FoamArgs a = args_for(cur, cur_hi, cur_pole, poles_virtual);
+        hipEvent_t t0 = nullptr, t1 = nullptr;
+        if (timer.enabled) {
+            auto& ev = timer.next(stream);
+            t0 = ev.first;
+            t1 = ev.second;
+        }
+        const dim3 grid(multi_blocks), blk(kFoamMultiThreads);
+        if (rebase)
+            hipExtLaunchKernelGGL((foam_multi_kernel<true>), grid, blk, multi_lds, stream, t0, t1, 0, a, d_multi, k,
+                                  to_rebase);
+        else
+            hipExtLaunchKernelGGL((foam_multi_kernel<false>), grid, blk, multi_lds, stream, t0, t1, 0, a, d_multi, k,
+                                  to_rebase);
+        SF_HIP(hipGetLastError());
+        for (int s = 0; s < k; ++s) advance(s == to_rebase);
+        if (k % 2 == 0) {               // the launch flips the ping-pong buffers once
+            cur = 1 - cur;
+            cur_pole = 1 - cur_pole;
         }
     }
 
@@ -841,6 +1085,7 @@ struct Foam {
             pole_cap = pole_slots;
         }
         SF_HIP(hipStreamSynchronize(stream));
+        multi_plan();
         drop_graph();
     }
 
@@ -986,6 +1231,13 @@ struct Foam {
 
     void step(int n) {
         int done = 0;
+        while (multi_steps && done < n) {
+            // equal shares: 10 steps at 8 per launch go as 5 + 5
+            const int left = n - done, launches = (left + multi_steps - 1) / multi_steps;
+            const int k = (left + launches - 1) / launches;
+            step_multi(k);
+            done += k;
+        }
         if (!poles_virtual && done < n) {   // first step reads the stored pole rows
             step_direct();
             ++done;
@@ -1433,6 +1685,8 @@ extern "C" int sf_foam_set_steps_per_launch(sf_foam* f, int32_t steps) {
         Foam* fm = F(f);
         SF_REQUIRE(steps == 1 || fm->two_ok, SF_ERR_INVALID,
                    "two steps per launch need every bubble at least 4 x 8 cells");
+        fm->multi_allowed = false;
+        fm->multi_steps = 0;
         if (steps == fm->steps_per_launch) return;
         fm->steps_per_launch = steps;
         fm->drop_graph();
@@ -1462,6 +1716,7 @@ extern "C" int sf_foam_set_tile_shapes(sf_foam* f, const int32_t* shapes) {
         Foam* fm = F(f);
         fm->materialize();              // pole partials change layout with the shapes
         std::copy(shapes, shapes + 4, fm->variant_of_bucket);
+        fm->multi_allowed = false;      // asked for by shape: the streaming kernels
         fm->layout_items();
     });
 }

@@ -1,0 +1,75 @@
+"""Several steps per launch of small foams (foam_multi_kernel) against the
+one-step kernels, over grids at the edges of its rule, and against itself cut
+into other launches.
+
+Both run the same cell arithmetic; only the pole means differ, FP64 ring sums
+against float-float ones (2^-44 of h a step at 1024 columns), and through
+them the roundings of the low word (2^-48 of h): over 40 steps 2^-38 of h.
+Surfactant has no ring means: its values are the same bits but for cells that
+the thickness decides (none ruptures here)."""
+import numpy as np
+import pytest
+
+from soap_bubble_simulation_amd.foam import FoamBubble, FoamDrainage, foam_params
+
+pytestmark = pytest.mark.gpu
+
+FOAMS = {
+    "smallest": [(3, 2), (4, 8), (3, 10)],
+    "one": [(64, 128)],
+    "odd": [(17, 34), (40, 78), (63, 126), (5, 1002)],
+    "widest": [(12, 1024), (30, 1022)],
+    "tall": [(900, 24), (1200, 30)],
+    "two_blocks_per_cu": [(18 + k % 20, 36 + 2 * (k % 20)) for k in range(200)],
+    "streaming": [(64, 1026), (16, 32)],
+}
+
+
+def _foam(grids, seed=1):
+    rng = np.random.default_rng(seed)
+    bub = [FoamBubble(n_theta=a, n_phi=b, bubble_radius=float(rng.uniform(5e-3, 2e-2)),
+                      viscosity=float(rng.uniform(1e-3, 4e-3)), h0=5e-7) for a, b in grids]
+    fm = FoamDrainage(foam_params(), bub)
+    n = fm.length
+    fm.set_fields(5e-7 * (1.0 + 0.1 * rng.uniform(-1, 1, n)), 0.5 + 0.2 * rng.uniform(-1, 1, n))
+    return fm
+
+
+@pytest.mark.parametrize("name", list(FOAMS))
+def test_matches_one_step_launches(name):
+    multi, one = _foam(FOAMS[name]), _foam(FOAMS[name])
+    one.set_steps_per_launch(1)
+    for steps in (1, 2, 9, 28):
+        multi.step(steps)
+        one.step(steps)
+        (ha, ga), (hb, gb) = multi.fields(), one.fields()
+        assert np.all(np.abs(ha - hb) <= 2.0 ** -38 * np.abs(hb)), (name, steps)
+        assert np.array_equal(ga, gb), (name, steps)
+
+
+@pytest.mark.parametrize("name", ["smallest", "odd", "widest", "tall", "two_blocks_per_cu"])
+def test_cut_into_other_launches(name):
+    a, b = _foam(FOAMS[name]), _foam(FOAMS[name])
+    a.step(40)
+    for steps in (1, 7, 2, 13, 17):
+        b.step(steps)
+    assert all(np.array_equal(x, y) for x, y in zip(a.fields(), b.fields()))
+
+
+def test_held_bubbles_and_explicit_shapes():
+    grids = FOAMS["odd"]
+    multi, one = _foam(grids), _foam(grids)
+    one.set_tile_shapes([9, 9, 9, 9])
+    for fm in (multi, one):
+        fm.step(3)
+        fm.set_active(np.array([1, 0, 1, 0], bool))
+        fm.step(21)
+        fm.set_active(None)
+        fm.step(10)
+    (ha, ga), (hb, gb) = multi.fields(), one.fields()
+    assert np.all(np.abs(ha - hb) <= 2.0 ** -38 * np.abs(hb)) and np.array_equal(ga, gb)
+    held = _foam(grids)
+    before = held.split(held.fields()[0])[1]
+    held.set_active(np.array([1, 0, 1, 0], bool))
+    held.step(19)
+    assert np.array_equal(held.split(held.fields()[0])[1][1:-1], before[1:-1])
