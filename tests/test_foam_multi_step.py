@@ -73,3 +73,19 @@ def test_held_bubbles_and_explicit_shapes():
     held.set_active(np.array([1, 0, 1, 0], bool))
     held.step(19)
     assert np.array_equal(held.split(held.fields()[0])[1][1:-1], before[1:-1])
+
+
+@pytest.mark.parametrize("launch", ["default", 1, 2])
+def test_readers_leave_the_run_alone(launch):
+    """Fields and statistics read between steps: the same bits as one run."""
+    a, b = _foam(FOAMS["odd"][1:]), _foam(FOAMS["odd"][1:])
+    if launch != "default":
+        a.set_steps_per_launch(launch)
+        b.set_steps_per_launch(launch)
+    a.step(33)
+    for steps in (1, 5, 8, 3, 16):
+        b.step(steps)
+        first = b.fields()
+        b.stats()
+        assert all(np.array_equal(x, y) for x, y in zip(first, b.fields()))
+    assert all(np.array_equal(x, y) for x, y in zip(a.fields(), b.fields()))
