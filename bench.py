@@ -49,6 +49,7 @@ SPECTRAL_CYCLES_PER_SLOT = 22.0
 SPECTRAL_SLOT20_CYCLES = 4.0 / 21.0
 SPECTRAL_TAIL_BUDGET = 1e-5
 SPECTRAL_MAX_SKIP = 2
+SPECTRAL_SERIES_CELLS = 1 << 20   # grids from here on take the cosine series
 
 
 def spectral_skip(cmf):
@@ -708,8 +709,13 @@ def main():
     n_spec = C.c_int64()
     L.check(lib.sf_spectral_kernel_timing(ctx.handle, 1 if spectral else 0, C.byref(ms_spec),
                                           C.byref(n_spec)))
-    timed_pass(max(args.steps + args.steps % spl, 500))
+    timed_steps = max(args.steps + args.steps % spl, 500)
+    timed_pass(timed_steps)
     drain_ms, drain_n = ctx.kernel_timing(False)
+    # small grids take several steps per launch by themselves
+    multi = drain_n > 0 and timed_steps / drain_n > 2.5
+    if multi:
+        spl = timed_steps / drain_n
     L.check(lib.sf_spectral_kernel_timing(ctx.handle, 0, C.byref(ms_spec), C.byref(n_spec)))
 
     # Headline pass: exactly K steps, no per-launch events, synchronised on
@@ -742,7 +748,7 @@ def main():
     # a launch advances (two with temporal blocking, whose HBM traffic is
     # about 24 B per cell per launch: see `traffic` and `one_step`).
     achieved = spl * BYTES_PER_CELL_STEP * cells / (drain_ms * 1e-3) / 1e9
-    kernel = ("drainage_band2_kernel" if spl == 2 else
+    kernel = ("drainage_multi_kernel" if multi else "drainage_band2_kernel" if spl == 2 else
               # 16-row float4 bands at 2048 x 4096, the scalar kernel with one
               # row per block at 128 x 256 (grids of up to 262144 cells)
               "drainage_band_kernel" if n_theta >= 1024 else "drainage_step_kernel")
@@ -785,8 +791,15 @@ def main():
         "state": {"min_h": stats.min_thickness, "max_h": stats.max_thickness,
                   "mass_m3": stats.mass, "time_s": stats.current_time, "finite": finite},
     }
-    if spectral and ms_spec.value:
-        # The spectral pass is bound by vector-ALU issue (two transcendentals
+    if spectral and ms_spec.value and cells >= SPECTRAL_SERIES_CELLS:
+        # Large grids take the cosine series: 28 B per cell (film state and
+        # view geometry in, three planes out) against the HBM peak.
+        achieved = cells * 28 / (ms_spec.value * 1e-3) / 1e9
+        out["kernels"]["spectral_hbm"] = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS,
+                                          "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
+                                          "model": "28 B per cell: hi, lo 8, view table 8, RGB 12"}
+    elif spectral and ms_spec.value:
+        # The direct spectral pass is bound by vector-ALU issue (two transcendentals
         # per slot; its MFMAs take a small share): its fraction of the
         # issue-model peak.
         skip = spectral_skip(cmf)
