@@ -330,10 +330,10 @@ struct SpecArgs {
     // from hpole, as materialize_poles_kernel would write it.
     const float2* hpole;
     int pole_virtual, nt, ntiles;
-    // Per-cell (q, optical path per thickness) of the current camera and film
-    // index: F = 4 q / (1 - q)^2, opd = h view.y in nm for h in m.  The
-    // geometry is fixed while they are, so spectral_view_kernel computes it
-    // once.
+    // Per-cell (q or F, optical path per thickness) of the current camera and
+    // film index: view.x is q up to kSerMaxQ, with F = 4 q / (1 - q)^2, else F
+    // itself (22 and more); opd = h view.y in nm for h in m.  The geometry is
+    // fixed while they are, so spectral_view_kernel computes it once.
     const float2* view;
 };
 
@@ -351,9 +351,13 @@ __device__ inline void spec_cell_ij(const SpecArgs& a, size_t cc, float inv_np, 
     if (j >= a.np) { ++i; j -= a.np; }
 }
 
-// q and cos theta_t of cell (i, j) at its view angle: q is the reflectance R
-// where F = 4 R / (1 - R)^2 is not clamped (interference_lut.rs:66-70 keeps
-// 1 - R at 1e-3 or more), else the root of 4 q / (1 - q)^2 = F.
+// q past which the cosine series is not used: kSerEps^(1 / 28), 28 terms.
+constexpr float kSerMaxQ = 0.6577f;
+
+// view.x and cos theta_t of cell (i, j) at its view angle: the reflectance R
+// as q where it is at most kSerMaxQ, else F = 4 R / (1 - R)^2 with 1 - R kept
+// at 1e-3 or more (interference_lut.rs:66-70).  F is stored and not a q that
+// gives it: 1 - q has lost ten bits where it is 1e-3.
 __device__ inline void spec_view_terms(const SpecArgs& a, int i, int j, float& q, float& cos_t_out) {
     const float4 rw = a.rows[i];
     const float2 cl = a.cols[j];
@@ -369,18 +373,15 @@ __device__ inline void spec_view_terms(const SpecArgs& a, int i, int j, float& q
     const float rs = (cos_i - a.n_film * cos_t) * __builtin_amdgcn_rcpf(fmaxf(cos_i + a.n_film * cos_t, 1e-4f));
     const float rp = (a.n_film * cos_i - cos_t) * __builtin_amdgcn_rcpf(fmaxf(a.n_film * cos_i + cos_t, 1e-4f));
     const float R = (rs * rs + rp * rp) * 0.5f;
-    q = R;
-    if (1.f - R < 1e-3f) {
-        const float s = sqrtf(1.f + 4e6f * R);
-        q = (s - 1.f) / (s + 1.f);
-    }
+    const float omr = fmaxf(1.f - R, 1e-3f);
+    q = R <= kSerMaxQ ? R : 4.f * R * __builtin_amdgcn_rcpf(omr * omr);
     cos_t_out = cos_t;
 }
 
-// Coefficient of finesse of a cell's q.
+// Coefficient of finesse of a cell's view.x.
 __device__ inline float spec_finesse(float q) {
     const float d = 1.f - q;
-    return 4.f * q * __builtin_amdgcn_rcpf(d * d);
+    return q <= kSerMaxQ ? 4.f * q * __builtin_amdgcn_rcpf(d * d) : q;
 }
 
 // Per-cell terms of the Airy sum: coefficient of finesse F and optical path
@@ -699,8 +700,6 @@ constexpr size_t kSerMinCells = size_t{1} << 20;
 // terms past the table: 141 against 143).
 constexpr double kSerMinTerms = 6.0;
 constexpr size_t kListBlocks = 1280;  // five waves per SIMD, all resident
-// q past which the wavelength sum is used: kSerEps^(1 / 28), 28 terms.
-constexpr float kSerMaxQ = 0.6577f;
 
 struct SeriesArgs {
     const float4* tab;      // [3 colours][kSerNodes] cubic coefficients of 2 G_c / 81

@@ -457,3 +457,35 @@ def test_spectral_series_state_and_curves(oracle):
         got = spectral_rgb(ctx, cam, cm)
     again = spectral_rgb(ctx, cam, cm)
     assert np.array_equal(got, again)
+
+
+@pytest.mark.parametrize("cos_i", [1e-5, 3e-5, 5e-5, 7e-5, 9e-5, 1.25e-4, 1.45e-4])
+def test_spectral_grazing_finesse(oracle, cos_i):
+    """Cells seen so close to grazing that 1 - R is clamped at 1e-3 (F about
+    4e6), through curves of one line of +1 and one of -1: the constant term
+    cancels, and what is left is (r(780) - r(380)) / 81 of r = 1 / (1 + F
+    cos^2), in proportion to 1 / F.  Its error, relative to the larger term:
+    2^-17 of the operand pair, 1e-5 of the phases (2^-22 revolutions at a
+    cosine of 0.33) and a few roundings of F, 3e-5 together."""
+    nt, npf, i = 33, 16, 11
+    p = L.Params()
+    L.check(L.lib().sf_params_cpu_default(p))
+    ctx = DrainageContext(p, nt, npf, 85e-9)
+    theta = i * math.pi / (nt - 1)
+    cam = (0.0, p.bubble_radius / math.cos(theta) * (1.0 + cos_i * math.tan(theta)), 0.0)
+    cm = np.zeros((81, 3), np.float32)
+    cm[0], cm[80] = 1.0, -1.0
+    L.check(L.lib().sf_spectral_set_operand(ctx.handle, L.SPECTRAL_OPERAND_BF16_PAIR))
+    got = spectral_rgb(ctx, cam, cm).reshape(3, nt, npf)[:, i]
+    cells = i * npf + np.arange(npf)
+    h = ctx.fields()[0]
+    lines = np.zeros_like(cm)
+    lines[0] = 1.0
+    # the oracle sums 1 - r: one line at a time, r = 1 - 81 rgb
+    r380 = 1.0 - 81.0 * oracle.spectral_cells(h, cells, p.bubble_radius, cam, 1.33, lines.astype(np.float64))
+    want = oracle.spectral_cells(h, cells, p.bubble_radius, cam, 1.33, cm.astype(np.float64))
+    scale = np.abs(r380).max() / 81.0
+    assert 1e-6 < 81.0 * scale < 4e-6
+    err = np.max(np.abs(got.T - want)) / scale
+    print("grazing cos %.3g: error of r %.2e" % (cos_i, err))
+    assert err <= 3e-5
