@@ -271,9 +271,10 @@ typedef struct sf_camera {
  *   rgb[c][cell] = (1/81) sum_k I_k cmf[k][c].
  * On grids of 2^20 cells and more with films up to about 2 um the sum is
  * evaluated, in the AUTO format, as a cosine series in the phase (FP32, each
- * channel within 2e-5 sum_k |cmf[k][c]| / 81 of the sum over the
- * wavelengths); the contraction then serves cells seen within about 3
- * degrees of grazing.
+ * channel within 4e-5 sum_k |cmf[k][c]| / 81 of the sum over the
+ * wavelengths in 64 bits: at most 1e-5 of terms left out and 2e-5 of the
+ * table for light at 380 nm, the rest FP32 rounding); the contraction then
+ * serves cells seen within about 3 degrees of grazing.
  * Operand format (sf_spectral_set_operand): by default FP16 when its
  * rounding of the reflectance moves no channel by more than 2.5e-4
  * (2^-18 sum_k |cmf[k][c]|) and the curves fit FP16, else a BF16 hi/lo

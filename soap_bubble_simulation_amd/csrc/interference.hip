@@ -677,6 +677,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
 // takes the sum over the wavelengths for them.  Cells whose terms leave the
 // table (thick films) take that sum in place (series_direct).
 //
+// Over every cell of the series (films to 1.9 um) the error relative to S_c /
+// 81 was at most 2.4e-5 for a line at 380 nm, 1.7e-5 at 450 nm and 1.3e-5 for
+// smooth curves, 2.7e-6, 1.7e-6 and 1e-6 in the mean square; the wavelength
+// sum has up to 3.1e-4 in FP16 and 2.0e-5 to 3.2e-5 with the BF16 pair.
+//
 // 2048 x 4096: 78 us (series 50, listed cells 23, the launches between them
 // 5) against 140 us for the wavelength sum everywhere (spectral_kernel); the
 // largest RGB error 2.5e-5 against 4.5e-5.  Of the series' 50 us, 43 are what

@@ -489,3 +489,31 @@ def test_spectral_grazing_finesse(oracle, cos_i):
     err = np.max(np.abs(got.T - want)) / scale
     print("grazing cos %.3g: error of r %.2e" % (cos_i, err))
     assert err <= 3e-5
+
+
+@pytest.mark.parametrize("film", [0.3e-6, 0.9e-6, 1.9e-6])
+def test_spectral_series_stated_bound(oracle, film):
+    """The header's bound on the series, 4e-5 of the mean |cmf|, at every cell
+    of 0.3 < q <= 0.6577 (where the terms left out and the table's share are
+    largest), for one line at 380 nm, whose table error is the largest."""
+    nt, npf = 1024, 1024
+    ctx, h0, p, cam, _ = _spectral_case(nt, npf, 5)
+    rng = np.random.default_rng(0)
+    h = h0 * (film / h0.max()) * rng.uniform(0.02, 1.0, h0.shape)
+    ctx.set_fields(h, np.full_like(h, 0.5))
+    h = ctx.fields()[0]
+    th = np.arange(nt)[:, None] * math.pi / (nt - 1)
+    ph = np.arange(npf)[None, :] * 2.0 * math.pi / npf
+    n = np.stack([np.sin(th) * np.cos(ph), np.broadcast_to(np.cos(th), (nt, npf)), np.sin(th) * np.sin(ph)], -1)
+    v = np.array(cam) - p.bubble_radius * n
+    ci = np.abs((v * n).sum(-1)) / np.linalg.norm(v, axis=-1)
+    ct = np.sqrt(1.0 - (1.0 - ci * ci) / 1.33 ** 2)
+    q = (((ci - 1.33 * ct) / (ci + 1.33 * ct)) ** 2 + ((1.33 * ci - ct) / (1.33 * ci + ct)) ** 2) / 2.0
+    cells = np.flatnonzero((q > 0.3) & (q < 0.6576))
+    assert cells.size > 20000
+    cm = np.zeros((81, 3), np.float32)
+    cm[0] = 1.0
+    want = oracle.spectral_cells(h, cells, p.bubble_radius, cam, 1.33, cm.astype(np.float64))
+    err = np.abs(spectral_rgb(ctx, cam, cm).reshape(3, -1)[:, cells].T - want) * 81.0
+    print("film %.1f um, line at 380 nm: max %.2e" % (film * 1e6, err.max()))
+    assert err.max() <= 4e-5
