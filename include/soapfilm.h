@@ -270,7 +270,7 @@ typedef struct sf_camera {
  * cmf[81][3] on 16-bit MFMA with FP32 accumulation:
  *   rgb[c][cell] = (1/81) sum_k I_k cmf[k][c].
  * On grids of 2^20 cells and more with films up to about 2 um the sum is
- * evaluated, in the AUTO format, as a cosine series in the phase (FP32, each
+ * evaluated, where the AUTO format is FP16, as a cosine series in the phase (FP32, each
  * channel within 4e-5 sum_k |cmf[k][c]| / 81 of the sum over the
  * wavelengths in 64 bits: at most 1e-5 of terms left out and 2e-5 of the
  * table for light at 380 nm, the rest FP32 rounding); the contraction then

@@ -517,3 +517,29 @@ def test_spectral_series_stated_bound(oracle, film):
     err = np.abs(spectral_rgb(ctx, cam, cm).reshape(3, -1)[:, cells].T - want) * 81.0
     print("film %.1f um, line at 380 nm: max %.2e" % (film * 1e6, err.max()))
     assert err.max() <= 4e-5
+
+
+@pytest.mark.parametrize("scale", [1.0, 100.0])
+def test_spectral_large_grid_operand_choice(oracle, scale):
+    """The automatic choice on a grid of the cosine series: curves whose FP16
+    bound passes 2.5e-4 take the operand pair there as everywhere (the same
+    bits), others the series.  Against 64 bits: the choice's budget of 2.5e-4
+    and, for curves of this mean, 2e-5 of it for the pair and FP32."""
+    nt, npf = 1024, 1024
+    ctx, h0, p, cam, cmf = _spectral_case(nt, npf, 33)
+    cm = (cmf * scale).astype(np.float32)
+    got = {}
+    for kind in (L.SPECTRAL_OPERAND_BF16_PAIR, L.SPECTRAL_OPERAND_AUTO):
+        L.check(L.lib().sf_spectral_set_operand(ctx.handle, kind))
+        got[kind] = spectral_rgb(ctx, cam, cm)
+    used = C.c_int32(-1)
+    L.check(L.lib().sf_spectral_get_operand(ctx.handle, C.byref(used)))
+    assert used.value == (L.SPECTRAL_OPERAND_FP16 if scale == 1.0 else L.SPECTRAL_OPERAND_BF16_PAIR)
+    same = np.array_equal(got[L.SPECTRAL_OPERAND_AUTO], got[L.SPECTRAL_OPERAND_BF16_PAIR])
+    assert same == (scale != 1.0)
+    cells = np.random.default_rng(2).choice(nt * npf, 20000, replace=False)
+    want = oracle.spectral_cells(ctx.fields()[0], cells, p.bubble_radius, cam, 1.33, cm.astype(np.float64))
+    err = np.max(np.abs(got[L.SPECTRAL_OPERAND_AUTO].reshape(3, -1)[:, cells].T - want), axis=0)
+    mean = np.abs(cm.astype(np.float64)).mean(axis=0)
+    print("operand choice, curves x %g: max err %s, of the mean %s" % (scale, err, err / mean))
+    assert np.all(err <= 2.5e-4 + 2e-5 * mean)
