@@ -739,6 +739,11 @@ struct Fno {
         return !(C % 16 || (2 * Mt) % 16 || T % 16 || kThetaThreads % (2 * C) || theta_fused_lds() > 64 * 1024);
     }
 
+    // Inference keeps activations between layers in 16 bits at n_phi 512 and
+    // 128.  n_phi = 256 runs the training pass's kernels instead: activations
+    // in FP32 and the lift formed in FP32, which its outputs always had.
+    bool inference16() const { return P != 256; }
+
     // Kernel paths the forward passes take at this shape (SF_FNO_PATH_* bits).
     int paths() const {
         int row_threads = 0, p = 0;
@@ -746,8 +751,8 @@ struct Fno {
             p |= SF_FNO_PATH_FUSED_ROWS;
             if (static_cast<size_t>(P * kCin + 2 * Mp * (kCin + 1)) * sizeof(float) <= 64 * 1024 && P <= kLiftDftMaxP)
                 p |= SF_FNO_PATH_LIFT_DFT;
-            if (theta_fused_ok()) p |= SF_FNO_PATH_FUSED_THETA;
-            if (row_wave_kernel()) p |= SF_FNO_PATH_WAVE_ROWS;
+            if (inference16() && theta_fused_ok()) p |= SF_FNO_PATH_FUSED_THETA;
+            if (inference16() && row_wave_kernel()) p |= SF_FNO_PATH_WAVE_ROWS;
         }
         return p;
     }
@@ -794,7 +799,7 @@ struct Fno {
         const long long R = static_cast<long long>(B) * N;
         int row_threads = 256;
         const RowKernel rk = row_kernel(&row_threads);
-        if (rk && !training) {
+        if (rk && !training && inference16()) {
             // Inference: the lift is folded into the layer-0 phi DFT and the
             // layer-0 row kernel, and the projection into the last one, so
             // neither x_0 nor x_L is written or read.
@@ -828,13 +833,13 @@ struct Fno {
         if (rk) {
             // The lift is folded into the first phi DFT and the first row
             // kernel, the projection into the last; every layer keeps its
-            // pre-activations and its output (FP32) for the backward pass.
+            // output in FP32 and, for the backward pass, its pre-activations.
             lift_dft(B);
             for (int l = 0; l < L; ++l) {
                 theta_stage(l, B);
                 const bool last = l == L - 1;
-                RowArgs ra{xs[l], Z, w + o_w[l], w + o_b[l], Iphi16, Ephi16, xs[l + 1], zs[l], last ? nullptr : X1,
-                           last ? 0 : 1, l == 0 ? in : nullptr, w + o_wl, w + o_bl, w + o_q, w + o_qb,
+                RowArgs ra{xs[l], Z, w + o_w[l], w + o_b[l], Iphi16, Ephi16, xs[l + 1], training ? zs[l] : nullptr,
+                           last ? nullptr : X1, last ? 0 : 1, l == 0 ? in : nullptr, w + o_wl, w + o_bl, w + o_q, w + o_qb,
                            last ? out : nullptr, 0};
                 hipLaunchKernelGGL(rk, dim3(static_cast<unsigned>(B * T)), dim3(row_threads), 0, stream, ra);
                 SF_HIP(hipGetLastError());

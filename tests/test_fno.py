@@ -223,6 +223,29 @@ def test_gpu_fused_activation_gradient_precision():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("width,modes_phi,layers", [(32, 16, 3), (16, 8, 2), (32, 8, 1)])
+def test_gpu_inference_at_256_columns_keeps_fp32(width, modes_phi, layers):
+    """n_phi = 256 keeps its activations between layers in FP32 and forms the
+    lift in FP32, in inference as in training: the loss against the inference
+    output is zero, where 16-bit activations put the two 1e-3 apart."""
+    from soap_bubble_simulation_amd import _lib as L
+    from soap_bubble_simulation_amd.surrogate import FnoSurrogate
+    m = FnoSurrogate(n_theta=32, n_phi=256, width=width, modes_theta=8, modes_phi=modes_phi, layers=layers, window=4,
+                     max_batch=2)
+    assert m.kernel_paths() == L.FNO_PATH_FUSED_ROWS | L.FNO_PATH_LIFT_DFT
+    s = R.Shapes.of(m.config)
+    flat, x, _ = rand_problem(s, 2, seed=12, scale=0.25)
+    f32, x32 = flat.astype(np.float32), x.astype(np.float32)
+    m.set_params(f32)
+    out = m.forward(x32)
+    ref, _, _ = R.forward(f32.astype(np.float64), x32.astype(np.float64), s)
+    print("n_phi 256 inference: rel", rel(out, ref))
+    assert rel(out, ref) <= 2e-2, rel(out, ref)
+    assert m.gradient(x32, out)[0] == 0.0
+    m.close()
+
+
+@pytest.mark.gpu
 def test_gpu_train_step_reduces_loss(model):
     s = R.Shapes.of(model.config)
     rng = np.random.default_rng(7)
