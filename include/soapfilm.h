@@ -208,10 +208,15 @@ int sf_drainage_kernel_timing(sf_drainage* ctx, int32_t enable, double* avg_ms,
  * and more (1024 x 2048 and up), 1 below.  On grids with n_phi <= 1024 and
  * few rows (1500 x 1024, 4000 x 256) sf_drainage_step takes up to 8 steps
  * per launch by itself, for all flags, with the same cell arithmetic and
- * pole rows formed in FP64; setting 1 here switches that off.
+ * pole rows formed in FP64; a run's results there do not depend on how its
+ * steps are grouped into calls, rendered steps included.  They differ from
+ * the streaming kernels' by FP32 rounding of the increments.  A call here
+ * with 1 or 2, also with the value got before, selects the streaming kernels
+ * for the rest of the context's life.
  * sf_drainage_get_steps_per_launch returns 1 or 2, what the launches of the
- * streaming kernels take; sf_drainage_kernel_timing then
- * averages over all its launches, of one or two steps.
+ * streaming kernels take (a small grid's own launches are not counted in);
+ * sf_drainage_kernel_timing averages over all launches, whatever steps each
+ * takes.
  * sf_drainage_step_spectral renders both states of a two-step launch: the
  * launch also writes the state between its steps.  No counterpart in the
  * reference, whose step dispatches one compute pass per step

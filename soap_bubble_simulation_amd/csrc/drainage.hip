@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256) void diag_finalize_kernel(const double2* part,
                 pole_mass_fixed, hist, slot, red_d);
 }
 
-// The history entries of a drainage_multi_kernel launch: block k folds step
+// The history entries of drainage_multi_kernel's steps: block k folds step
 // k's per-block partials (the pole rows are in them unless copied through).
 __global__ __launch_bounds__(64) void multi_diag_kernel(const double2* part, int nblocks, double fixed, double2* hist,
                                                         int slot0, int cap) {
@@ -445,7 +445,7 @@ Drainage::~Drainage() {
 // 6.7 | 7.9 -> 9.2, hence kMultiMaxCols.
 void Drainage::multi_plan() {
     constexpr int kCus = 256;
-    constexpr size_t kLdsBytes = 150 * 1024;
+    constexpr size_t kLdsBytes = 128 * 1024;      // beside 28 KB of static arrays
     if (nt < 3 || np > kMultiMaxCols) return;
     multi_rows = (nt - 2 + kCus - 1) / kCus;
     if (multi_rows > kMultiRows) return;
@@ -729,9 +729,16 @@ void Drainage::materialize_poles() {
     poles_virtual = false;
 }
 
-// Reduces the per-block FP64 partials of the last diagnosed step, which no
+// Reduces the per-block FP64 partials of the last diagnosed steps, which no
 // later launch has consumed yet.
 void Drainage::finalize_diag() {
+    if (multi_pending > 0) {
+        hipLaunchKernelGGL(multi_diag_kernel, dim3(multi_pending), dim3(64), 0, stream, multi_part,
+                           static_cast<int>(cdiv(nt - 2, multi_rows)), multi_fixed, diag_hist, multi_slot,
+                           static_cast<int>(kHistCap));
+        SF_HIP(hipGetLastError());
+        multi_pending = 0;
+    }
     for (int q = 0; q < npending; ++q) {
         const PendingDiag& e = pending[q];
         hipLaunchKernelGGL(diag_finalize_kernel, dim3(1), dim3(256), 0, stream, diag_part[e.buf], e.nblocks,
@@ -933,7 +940,7 @@ void Drainage::launch_two(double dt, bool with_mid) {
     steps_taken += 2;
 }
 
-// k steps in one launch of drainage_multi_kernel (2 <= k <= multi_steps).
+// k steps in one launch of drainage_multi_kernel (1 <= k <= multi_steps).
 void Drainage::launch_multi(double dt, int k) {
     const bool marangoni = (p.flags & SF_FLAG_MARANGONI) != 0;
     const bool surfactant = (p.flags & SF_FLAG_SURFACTANT) != 0;
@@ -947,7 +954,6 @@ void Drainage::launch_multi(double dt, int k) {
     fill_common_args(m.s, static_cast<float>(dt));
     m.steps = k;
     m.rows = multi_rows;
-    m.inv_np = 1.0 / np;
     for (int s = 0; s < k; ++s) {
         StepArgs one{};
         schedule_fronts(dt, one);
@@ -981,9 +987,17 @@ void Drainage::launch_multi(double dt, int k) {
     a.gpole_in = gpole[cur_pole];
     a.hpole_out = hpole[1 - cur_pole];
     a.gpole_out = gpole[1 - cur_pole];
-    finalize_diag();
-    if (diag && !multi_part) multi_part = dalloc<double2>(static_cast<size_t>(kMultiSteps) * blocks);
-    m.part = multi_part;
+    const double fixed = h_avg ? 0.0 : pole_mass_fixed;
+    const int slot = static_cast<int>(hist_count % kHistCap);
+    // Up to kMultiSteps diagnosed steps wait for one fold: a fold after every
+    // launch took 1.7 of a rendered step's 15.0 us at 128 x 256.
+    if (!diag || npending > 0 || multi_pending + k > kMultiSteps || fixed != multi_fixed ||
+        slot != (multi_slot + multi_pending) % static_cast<int>(kHistCap))
+        finalize_diag();
+    if (diag) {
+        if (!multi_part) multi_part = dalloc<double2>(static_cast<size_t>(kMultiSteps) * blocks);
+        m.part = multi_part + static_cast<size_t>(multi_pending) * blocks;
+    }
     const size_t bytes = static_cast<size_t>(multi_rows + 2 * k) * np * (gmode ? 12 : 8);
     const MultiFn fn = multi_fn(gmode, marangoni, diag);
     if (bytes > 64 * 1024)
@@ -997,10 +1011,9 @@ void Drainage::launch_multi(double dt, int k) {
     }
     SF_HIP(hipGetLastError());
     if (diag) {
-        hipLaunchKernelGGL(multi_diag_kernel, dim3(k), dim3(64), 0, stream, multi_part, static_cast<int>(blocks),
-                           h_avg ? 0.0 : pole_mass_fixed, diag_hist, static_cast<int>(hist_count % kHistCap),
-                           static_cast<int>(kHistCap));
-        SF_HIP(hipGetLastError());
+        if (multi_pending == 0) multi_slot = slot;
+        multi_fixed = fixed;
+        multi_pending += k;
         hist_count += k;
     }
     cur = 1 - cur;
@@ -1018,8 +1031,9 @@ void Drainage::step(int n_steps, double dt, bool flush) {
     dt = resolve_dt(dt);
     for (int s = 0; s < n_steps;) {
         const int left = n_steps - s;
-        if (multi_steps && left >= 2) {
-            // equal shares: 10 steps at 8 per launch go as 5 + 5
+        if (multi_steps) {
+            // equal shares: 10 steps at 8 per launch go as 5 + 5; a lone step
+            // too, so that the results do not depend on the grouping
             const int launches = (left + multi_steps - 1) / multi_steps, k = (left + launches - 1) / launches;
             launch_multi(dt, k);
             s += k;
@@ -1518,6 +1532,7 @@ extern "C" int sf_drainage_set_steps_per_launch(sf_drainage* ctx, int32_t steps)
     return guard([&] {
         SF_REQUIRE(ctx != nullptr, SF_ERR_INVALID, "ctx is NULL");
         SF_REQUIRE(steps == 1 || steps == 2, SF_ERR_INVALID, "steps per launch must be 1 or 2, got %d", steps);
+        D(ctx)->finalize_diag();
         D(ctx)->steps_per_launch = steps;
         D(ctx)->multi_steps = 0;
     });

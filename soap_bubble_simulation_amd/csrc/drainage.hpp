@@ -69,7 +69,9 @@ struct Drainage {
     // Several steps per launch on small grids (drainage_multi_kernel): rows
     // per block and the most steps, 0 where it is not used.
     int multi_rows = 1, multi_steps = 0;
-    double2* multi_part = nullptr;
+    double2* multi_part = nullptr;       // diagnostics of its steps not yet folded:
+    int multi_pending = 0, multi_slot = 0;      // how many, the first one's history slot,
+    double multi_fixed = 0.0;            // and the volume of copied pole rows
     // Field exchange with the host: FP64 staging (at most 2 kStageCells
     // cells, made at the first use), maxima per block, pole rows.
     static constexpr size_t kStageCells = size_t{1} << 21;

@@ -776,7 +776,10 @@ __device__ __forceinline__ void cell_step(const StepArgs& a, const RowF& rc, flo
 // block per CU or fewer rows, and fewer steps the wider the rows
 // (Drainage::multi_plan).  The ring sums are FP64 and go through DPP moves:
 // with LDS shuffles and a float-float tree they were 1 us of a step, front
-// boxes fetched per cell another 1 to 4 us.  us per step with thinning,
+// boxes fetched per cell another 1 to 4 us.  Ring sums run in column order
+// over fixed threads, diagnostics over the block's own cells, and a ring's
+// sum is a float pair inside a launch as between launches: a run does not
+// depend on how its steps are grouped into launches.  us per step with thinning,
 // one-step launches -> these: 128 x 256 5.2 -> 3.4, 256 x 512 5.2 -> 3.3,
 // 500 x 1003 (no vector path) 13.5 -> 4.5.
 constexpr int kMultiSteps = 8;
@@ -791,7 +794,6 @@ struct MultiArgs {
     int steps;                        // 1 .. kMultiSteps
     int rows;                         // rows a block owns, at most kMultiRows
     unsigned rebase;                  // bit k: step k renormalises hi, lo
-    double inv_np;
     int nf[kMultiSteps];
     FrontBox fr[kMultiSteps][kMaxFronts];
     double2* part;                    // diagnostics: [steps][blocks] {mass, max lambda}
@@ -845,6 +847,8 @@ __global__ __launch_bounds__(kMultiThreads) void drainage_multi_kernel(const Mul
     extern __shared__ __align__(16) float lds_state[];
     __shared__ float4 s_row[kMultiRowsAll];      // cot / (2 dth), 1 / (s^2 dph^2), dt coef sin, 1 / s
     __shared__ double s_ring[4][kWaves];         // ring sums per wave: h top, h bottom, g top, g bottom
+    __shared__ double s_pre[2][kMultiMaxCols];   // ring values of h before the fronts act
+    __shared__ float s_preg[GWRITE ? 2 : 1][GWRITE ? kMultiMaxCols : 1];
     __shared__ RowD s_rowd[DIAG ? kMultiRows : 1];
     __shared__ double s_mass[DIAG ? kMultiSteps : 1][kWaves], s_lam[DIAG ? kMultiSteps : 1][kWaves];
     const int np = a.np, nt = a.nt, tid = threadIdx.x;
@@ -879,7 +883,7 @@ __global__ __launch_bounds__(kMultiThreads) void drainage_multi_kernel(const Mul
             gmean[e] = g.x + g.y;
         }
     }
-    double total[2] = {0.0, 0.0}, gtotal[2] = {0.0, 0.0};
+    float2 total[2] = {make_float2(0.f, 0.f), make_float2(0.f, 0.f)}, gtotal[2] = {total[0], total[1]};
     // A thread's cells lie T apart in the step's rows; row and column of each
     // relative to the first row are the same in every step.
     int rel[kMultiCells], col[kMultiCells];
@@ -922,8 +926,6 @@ __global__ __launch_bounds__(kMultiThreads) void drainage_multi_kernel(const Mul
         }
         float2 nhl[kMultiCells];
         float ng[kMultiCells];
-        double ring[2] = {0.0, 0.0}, gring[2] = {0.0, 0.0};
-        double mass = 0.0, lam = 0.0;
 #pragma unroll
         for (int q = 0; q < kMultiCells; ++q) {
             if (q * T >= count) break;                                      // uniform
@@ -956,27 +958,19 @@ __global__ __launch_bounds__(kMultiThreads) void drainage_multi_kernel(const Mul
             // ring values before the fronts act (update_poles runs first)
             if (cap && in) {
                 const double hv = static_cast<double>(C.x) + static_cast<double>(lo_new);
-                if (i == 1) {
-                    ring[0] += hv;
-                    gring[0] += static_cast<double>(g_new);
-                }
-                if (i == nt - 2) {
-                    ring[1] += hv;
-                    gring[1] += static_cast<double>(g_new);
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    if (i != (e == 0 ? 1 : nt - 2)) continue;
+                    s_pre[e][j] = hv;
+                    if (GWRITE) s_preg[e][j] = g_new;
                 }
             }
             if (in && ((front >> q) & 1)) lo_new = front_thin(a, C.x, lo_new);
             nhl[q] = make_float2(C.x, lo_new);
             if (rebase) two_sum(C.x, lo_new, nhl[q].x, nhl[q].y);
             ng[q] = g_new;
-            if (DIAG && in && i >= r0 && i < r1) {
-                const RowD& rd = s_rowd[i - r0];
-                const double hv = static_cast<double>(C.x) + static_cast<double>(lo_new);
-                mass += hv * rd.area;
-                lam = fmax(lam, rd.lam_grid + a.coef3 * rd.sin_abs * hv * hv);
-            }
         }
-        __syncthreads();                         // every neighbour is read
+        __syncthreads();                         // every neighbour is read, the ring values are written
 #pragma unroll
         for (int q = 0; q < kMultiCells; ++q) {
             if (q * T >= count) break;
@@ -988,12 +982,13 @@ __global__ __launch_bounds__(kMultiThreads) void drainage_multi_kernel(const Mul
         if (cap) {
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
+                if (e == 0 ? u0 != 1 : u1 != nt - 1) continue;
                 if (a.h_pole_sum) {
-                    const double v = wave_sum(ring[e]);
+                    const double v = wave_sum(tid < np ? s_pre[e][tid] : 0.0);
                     if (lane == 0) s_ring[e][wave] = v;
                 }
                 if (GWRITE && a.g_pole_sum) {
-                    const double v = wave_sum(gring[e]);
+                    const double v = wave_sum(tid < np ? static_cast<double>(s_preg[GWRITE ? e : 0][GWRITE ? tid : 0]) : 0.0);
                     if (lane == 0) s_ring[2 + e][wave] = v;
                 }
             }
@@ -1006,26 +1001,40 @@ __global__ __launch_bounds__(kMultiThreads) void drainage_multi_kernel(const Mul
             for (int e = 0; e < 2; ++e) {
                 if (e == 0 ? u0 != 1 : u1 != nt - 1) continue;
                 if (a.h_pole_sum) {
-                    total[e] = lane_value(row_sum(lane < kWaves ? s_ring[e][lane] : 0.0), kWaves - 1);
-                    double v = total[e] * m.inv_np;
-                    v = fma(fma(-v, static_cast<double>(np), total[e]), m.inv_np, v);
-                    mean[e] = split_pair(v);
+                    total[e] = split_pair(lane_value(row_sum(lane < kWaves ? s_ring[e][lane] : 0.0), kWaves - 1));
+                    mean[e] = pole_mean_of_sum(total[e], a.np_f);
                 }
                 if (GWRITE && a.g_pole_sum) {
-                    gtotal[e] = lane_value(row_sum(lane < kWaves ? s_ring[2 + e][lane] : 0.0), kWaves - 1);
-                    gmean[e] = static_cast<float>(gtotal[e] * m.inv_np);
+                    gtotal[e] = split_pair(lane_value(row_sum(lane < kWaves ? s_ring[2 + e][lane] : 0.0), kWaves - 1));
+                    const float2 g = pole_mean_of_sum(gtotal[e], a.np_f);
+                    gmean[e] = g.x + g.y;
                 }
             }
         }
         have = have || a.h_pole_sum;
         ghave = ghave || (GWRITE && a.g_pole_sum);
         if (DIAG) {
+            // the block's own cells, whatever rows the step updates
+            const int from = (r0 - e0) * np, own = (r1 - r0) * np;
+            double mass = 0.0, lam = 0.0;
+#pragma unroll
+            for (int q = 0; q < kMultiCells; ++q) {
+                if (q * T >= own) break;                                    // uniform
+                if (tid + q * T >= own) continue;
+                const float2 v = HL[from + tid + q * T];
+                const RowD& rd = s_rowd[DIAG ? rel[q] : 0];
+                const double hv = static_cast<double>(v.x) + static_cast<double>(v.y);
+                mass += hv * rd.area;
+                lam = fmax(lam, rd.lam_grid + a.coef3 * rd.sin_abs * hv * hv);
+            }
             mass = wave_sum(mass);
             lam = wave_dmax(lam);
             if (lane == 0) {
                 if (a.h_pole_sum && wave == 0) {     // the owner of a ring adds its pole row
-                    if (r0 == 1) mass += a.pole_area_top * total[0];
-                    if (r1 == nt - 1) mass += a.pole_area_bot * total[1];
+                    if (r0 == 1)
+                        mass += a.pole_area_top * (static_cast<double>(total[0].x) + static_cast<double>(total[0].y));
+                    if (r1 == nt - 1)
+                        mass += a.pole_area_bot * (static_cast<double>(total[1].x) + static_cast<double>(total[1].y));
                 }
                 s_mass[k][wave] = mass;
                 s_lam[k][wave] = lam;
@@ -1046,9 +1055,8 @@ __global__ __launch_bounds__(kMultiThreads) void drainage_multi_kernel(const Mul
     for (int e = 0; e < 2; ++e) {
         if (e == 0 ? r0 != 1 : r1 != nt - 1) continue;
         for (int t = tid; t < a.ntiles; t += T) {
-            if (a.h_pole_sum) a.hpole_out[e * a.ntiles + t] = t == 0 ? split_pair(total[e]) : make_float2(0.f, 0.f);
-            if (GWRITE && a.g_pole_sum)
-                a.gpole_out[e * a.ntiles + t] = t == 0 ? split_pair(gtotal[e]) : make_float2(0.f, 0.f);
+            if (a.h_pole_sum) a.hpole_out[e * a.ntiles + t] = t == 0 ? total[e] : make_float2(0.f, 0.f);
+            if (GWRITE && a.g_pole_sum) a.gpole_out[e * a.ntiles + t] = t == 0 ? gtotal[e] : make_float2(0.f, 0.f);
         }
     }
     if (DIAG) {

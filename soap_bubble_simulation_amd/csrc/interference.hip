@@ -1497,7 +1497,11 @@ static void step_spectral(Drainage* d, int32_t n_steps, double dt, const sf_came
     // two steps go into one stencil launch, that launch also writes the
     // state between them, and both states are rendered.
     for (int s = 0; s < n_steps;) {
-        if (d->two_step_next(n_steps - s)) {
+        if (d->multi_steps) {           // the kernel sf_drainage_step takes, for the same results
+            d->launch_multi(dt, 1);
+            spectral_launch(d, cam, refractive_index, nullptr, d->stream, nullptr, frame(s));
+            s += 1;
+        } else if (d->two_step_next(n_steps - s)) {
             d->launch_two(dt, true);
             const FieldView mid{d->mid_hi, d->lo_mid, d->mid_hpole, !(d->p.flags & SF_FLAG_POLES_COPY_H)};
             spectral_launch(d, cam, refractive_index, nullptr, d->stream, &mid, frame(s));

@@ -1,5 +1,7 @@
 """Several steps per launch on small grids (drainage_multi_kernel) against the
 FP64 oracle and against one step per launch."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -97,23 +99,33 @@ def test_multi_step_matches_oracle(oracle, nt, npf, flags, rebase):
     assert np.linalg.norm(gc - go) <= 1e-5 * np.linalg.norm(go)
 
 
-def test_multi_step_call_patterns():
-    """Steps in any grouping give the same state: launches of 2 .. 8 steps,
-    single steps between them, and reads that write the pole rows out."""
-    nt, npf = 96, 200
-    p = _params(TFE | SURF)
+@pytest.mark.parametrize("nt,npf,flags,rebase", [
+    (96, 200, TFE | SURF, 8), (3, 7, TFE | SURF | DIAG, 8), (4, 8, TFE, 3), (12, 1024, MARA | SURF | AVG | DIAG, 8),
+    (129, 255, MARA | SURF | AVG | DIAG, 5), (128, 256, TFE | DIAG, 8), (300, 601, TFE | SURF | COPY | DIAG, 8),
+    (514, 1024, TFE | SURF | DIAG, 8), (1500, 1024, TFE | SURF, 8), (4000, 256, TFE | DIAG, 8)])
+def test_multi_step_call_patterns(nt, npf, flags, rebase):
+    """Steps in any grouping give the same bits, history included: launches of
+    1 .. 8 steps, reads that write the pole rows out between them, and steps
+    that are rendered one by one."""
+    p = _params(flags, rebase)
     h, g = _fields(nt, npf, 9)
+    cam = L.Camera()
+    for k, x in enumerate(W.camera(p.bubble_radius)):
+        cam.position[k] = x
+    cmf = W.spectral_cmf(2).astype(np.float32)
     ref = None
-    for groups in ([30], [1] * 30, [2, 3, 4, 5, 6, 7, 3], [8, 1, 8, 1, 8, 4], [29, 1]):
+    for groups in ([30], [1] * 30, [2, 3, 4, 5, 6, 7, 3], [8, 1, 8, 1, 8, 4], [29, 1], "rendered"):
         ctx = DrainageContext(p, nt, npf, 5e-7)
         ctx.set_fields(h, g)
         dt = 0.3 * ctx.stats().dt_cfl
-        for n in groups:
-            ctx.step(n, dt)
-            ctx.get_thickness(0.0, 0.0)
-        out = ctx.fields()
+        if groups == "rendered":
+            L.check(L.lib().sf_drainage_step_spectral(ctx.handle, 17, dt, C.byref(cam), 1.33, L.fptr(cmf)))
+            ctx.step(13, dt)
+        else:
+            for n in groups:
+                ctx.step(n, dt)
+                ctx.get_thickness(0.0, 0.0)
+        out = [*ctx.fields(), *ctx.history(30)]
         if ref is None:
             ref = out
-        scale = np.abs(ref[0] - h).max()
-        assert np.abs(out[0] - ref[0]).max() <= 2e-5 * scale, groups
-        assert np.abs(out[1] - ref[1]).max() <= 2e-6, groups
+        assert all(np.array_equal(x, y) for x, y in zip(out, ref)), groups
