@@ -965,6 +965,9 @@ struct Foam {
     // cells a block and step that keep one block per CU (two where one does
     // not fit), so that wide and narrow bubbles' blocks take alike;
     // sqrt(10^4 / n_phi) steps of the widest bubble, as Drainage::multi_plan.
+    // Whether the foam takes the kernel is a matter of all its bubbles, held
+    // ones included, so that a bubble's results do not depend on which others
+    // are stepped with it; fewer active ones only get smaller blocks.
     // us per step, one-step launches -> these: 6 bubbles of 16-24 latitudes
     // 3.9 -> 1.9, 100 of 24-48 5.3 -> 2.8, 16 of 64-256 8.0 -> 5.2; two blocks
     // per CU: 200 of 16-40 5.8 -> 4.9, 30 of 64-256 10.6 -> 8.8.  At three and
@@ -973,36 +976,47 @@ struct Foam {
     void multi_plan() {
         multi_steps = 0;
         int np = 0;
-        for (int b = 0; b < nb; ++b)
-            if (active[b]) np = std::max(np, bub[b].np);
-        if (!multi_allowed || np == 0 || np > kFoamMultiCols) return;
+        for (int b = 0; b < nb; ++b) np = std::max(np, bub[b].np);
+        if (!multi_allowed || np > kFoamMultiCols) return;
         const int k = std::max(2, std::min(static_cast<int>(std::lround(std::sqrt(1e4 / np))), kFoamMultiSteps));
-        auto blocks = [&](int cells) {
-            int64_t n = 0;
-            for (int b = 0; b < nb; ++b)
-                if (active[b]) n += (bub[b].nt - 2 + multi_rows(bub[b], k, cells) - 1) / multi_rows(bub[b], k, cells);
-            return n;
-        };
         constexpr int kMost = kFoamMultiCells * kFoamMultiThreads;
-        int most = n_cu;
-        while (most <= kFoamMultiBlocks * n_cu && blocks(kMost) > most) most += n_cu;
-        if (most > kFoamMultiBlocks * n_cu) return;
-        int lo = 0, hi_ = kMost;                   // least cells that fit, by bisection
-        while (hi_ - lo > 1) {
-            const int mid = (lo + hi_) / 2;
-            (blocks(mid) <= most ? hi_ : lo) = mid;
-        }
-        std::vector<FoamMultiItem> items;
+        // Least cells that keep a set of bubbles to its blocks, by bisection;
+        // 0 where kMost cells do not.
+        auto least = [&](bool all) {
+            auto blocks = [&](int cells) {
+                int64_t n = 0;
+                for (int b = 0; b < nb; ++b)
+                    if (all || active[b])
+                        n += (bub[b].nt - 2 + multi_rows(bub[b], k, cells) - 1) / multi_rows(bub[b], k, cells);
+                return n;
+            };
+            int most = n_cu;
+            while (most <= kFoamMultiBlocks * n_cu && blocks(kMost) > most) most += n_cu;
+            if (most > kFoamMultiBlocks * n_cu) return 0;
+            int lo = 0, hi_ = kMost;
+            while (hi_ - lo > 1) {
+                const int mid = (lo + hi_) / 2;
+                (blocks(mid) <= most ? hi_ : lo) = mid;
+            }
+            return hi_;
+        };
+        int cells = least(true);
+        if (cells == 0) return;
         size_t held = 0, updated = 0;
         for (int b = 0; b < nb; ++b) {
-            if (!active[b]) continue;
-            const FoamBubble& B = bub[b];
-            const int r = multi_rows(B, k, hi_);
-            for (int r0 = 1; r0 < B.nt - 1; r0 += r) items.push_back({b, r0, std::min(r0 + r, B.nt - 1), 0});
-            held = std::max(held, static_cast<size_t>(r + 2 * k) * B.np);
-            updated = std::max(updated, static_cast<size_t>(r + 2 * (k - 1)) * B.np);
+            const int r = multi_rows(bub[b], k, cells);
+            held = std::max(held, static_cast<size_t>(r + 2 * k) * bub[b].np);
+            updated = std::max(updated, static_cast<size_t>(r + 2 * (k - 1)) * bub[b].np);
         }
-        if (items.empty() || held * 12 > kFoamMultiLds || updated > static_cast<size_t>(kMost)) return;
+        if (held * 12 > kFoamMultiLds || updated > static_cast<size_t>(kMost)) return;
+        cells = std::min(cells, least(false));
+        std::vector<FoamMultiItem> items;
+        for (int b = 0; b < nb; ++b) {
+            if (!active[b]) continue;
+            const int r = multi_rows(bub[b], k, cells);
+            for (int r0 = 1; r0 < bub[b].nt - 1; r0 += r) items.push_back({b, r0, std::min(r0 + r, bub[b].nt - 1), 0});
+        }
+        if (items.empty()) return;
         if (static_cast<int>(items.size()) > multi_cap) {
             (void)hipFree(d_multi);
             d_multi = nullptr;
