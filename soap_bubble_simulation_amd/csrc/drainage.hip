@@ -412,6 +412,8 @@ Drainage::Drainage(const sf_params& prm, int n_theta, int n_phi) : p(prm), nt(n_
     diag_hist = dalloc<double2>(kHistCap);
     stats_part = dalloc<StatsPart>(kStatsBlocks);
     stats_out = dalloc<StatsPart>(1);
+    stage = dalloc<double>(2 * std::min(n, kStageCells));
+    if (multi_steps) multi_part = dalloc<double2>(static_cast<size_t>(kMultiSteps) * cdiv(nt - 2, multi_rows));
     split_part = dalloc<float>(kSplitBlocks);
     pole_rows = dalloc<float>(4 * static_cast<size_t>(np) + 1);
     tables_dirty = true;
@@ -509,19 +511,13 @@ void Drainage::update_fixed_pole_mass(bool with_max) {
     if (with_max) h_max = r[4 * w];
 }
 
-// Two fields' worth of kStageCells FP64 cells, at most.
-double* Drainage::ensure_stage() {
-    if (!stage) stage = dalloc<double>(2 * std::min(n, kStageCells));
-    return stage;
-}
-
 // Sets the fields from host arrays (nullptr: keeps one), in both ping-pong
 // halves so that rows a step never writes (the poles, and Γ when it is
 // frozen) hold the same values in both.
 template <class T>
 void Drainage::upload(const T* h, const T* gam) {
     constexpr bool wide = sizeof(T) == 8;
-    double* const st = wide && (h || gam) ? ensure_stage() : nullptr;
+    double* const st = stage;
     const size_t chunk = wide ? std::min(n, kStageCells) : n;
     if (!h) {
         hipLaunchKernelGGL(split_h_kernel<From::kState>, dim3(kSplitBlocks), dim3(256), 0, stream, nullptr, hi[cur_hi],
@@ -561,7 +557,7 @@ void Drainage::upload(const T* h, const T* gam) {
 // The current fields into host arrays (nullptr: not wanted).
 template <class T>
 void Drainage::download(T* h, T* gam) {
-    T* const st = reinterpret_cast<T*>(ensure_stage());
+    T* const st = reinterpret_cast<T*>(stage);
     const size_t chunk = std::min(n, kStageCells);
     for (size_t c = 0; c < n; c += chunk) {
         const size_t m = std::min(chunk, n - c);
@@ -994,10 +990,7 @@ void Drainage::launch_multi(double dt, int k) {
     if (!diag || npending > 0 || multi_pending + k > kMultiSteps || fixed != multi_fixed ||
         slot != (multi_slot + multi_pending) % static_cast<int>(kHistCap))
         finalize_diag();
-    if (diag) {
-        if (!multi_part) multi_part = dalloc<double2>(static_cast<size_t>(kMultiSteps) * blocks);
-        m.part = multi_part + static_cast<size_t>(multi_pending) * blocks;
-    }
+    if (diag) m.part = multi_part + static_cast<size_t>(multi_pending) * blocks;
     const size_t bytes = static_cast<size_t>(multi_rows + 2 * k) * np * (gmode ? 12 : 8);
     const MultiFn fn = multi_fn(gmode, marangoni, diag);
     if (bytes > 64 * 1024)

@@ -73,8 +73,9 @@ struct Drainage {
     int multi_pending = 0, multi_slot = 0;      // how many, the first one's history slot,
     double multi_fixed = 0.0;            // and the volume of copied pole rows
     // Field exchange with the host: FP64 staging (at most 2 kStageCells
-    // cells, made at the first use), maxima per block, pole rows.
-    static constexpr size_t kStageCells = size_t{1} << 21;
+    // cells, 8 MB), maxima per block, pole rows.  Made with the context: a
+    // reader of a card that has filled up since allocates nothing.
+    static constexpr size_t kStageCells = size_t{1} << 19;
     static constexpr int kSplitBlocks = 512;
     double* stage = nullptr;
     float* split_part = nullptr;
@@ -175,7 +176,6 @@ struct Drainage {
     void upload(const T* h, const T* gam);
     template <class T>
     void download(T* h, T* gam);
-    double* ensure_stage();
     void fill(double h0, double gamma0);
     void front_columns(HostFront& f) const;
     void spawn_front();

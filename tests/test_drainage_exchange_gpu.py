@@ -1,6 +1,8 @@
 """Fields and history between host and device: the FP64 split into two FP32
-words and back, both in pieces of 2^21 cells, kept fields, and a history ring
+words and back, both in pieces of 2^19 cells, kept fields, and a history ring
 that has wrapped."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -19,7 +21,7 @@ def _context(nt, npf, flags=0, rebase=None):
     return DrainageContext(p, nt, npf, 5e-7)
 
 
-@pytest.mark.parametrize("nt,npf", [(3, 1), (5, 7), (64, 128), (257, 511), (1499, 1399), (1500, 1401), (2048, 2048)])
+@pytest.mark.parametrize("nt,npf", [(3, 1), (5, 7), (64, 128), (257, 511), (1024, 512), (1025, 512), (1499, 1399), (1500, 1401), (2048, 2048)])
 def test_fields_round_trip(nt, npf):
     rng = np.random.default_rng(nt)
     h = rng.uniform(1e-7, 9e-7, (nt, npf))
@@ -81,3 +83,29 @@ def test_history_ring_wraps():
     short = c.history(130)
     assert np.array_equal(short[0], last[0][-130:]) and np.array_equal(short[1], last[1][-130:])
     assert len(c.history(0)[0]) == 0
+
+
+@pytest.mark.parametrize("nt,npf,flags", [(1500, 1024, 0), (1024, 2048, 0), (4000, 256, 32 | 8)])
+def test_exchange_and_steps_allocate_nothing(nt, npf, flags):
+    """Device memory is taken when a context is made: exchanging its fields,
+    stepping it and reading its history take none, so they cannot fail on a
+    card that has filled up since."""
+    hip = C.CDLL("libamdhip64.so.7")
+
+    def free():
+        a, b = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        return a.value
+
+    warm = _context(nt, npf, flags)        # code objects and the runtime's own buffers
+    for c in (warm, _context(nt, npf, flags)):
+        before = free()
+        h = np.full((nt, npf), 5e-7)
+        c.fields()
+        c.fields_f32()
+        c.set_fields(h, None)
+        c.set_fields_f32(h.astype(np.float32), None)
+        c.step(9, 1e-9)
+        c.history(4)
+        after = free()
+    assert after == before
