@@ -1644,15 +1644,16 @@ extern "C" int sf_foam_set_fields_f64(sf_foam* f, const double* h, const double*
                 hh[c] = static_cast<float>(h[c]);
                 ll[c] = static_cast<float>(h[c] - static_cast<double>(hh[c]));
             }
-        } else {
-            SF_HIP(hipMemcpy(hh.data(), fm->hi[fm->cur_hi], fm->total * 4, hipMemcpyDeviceToHost));
-            SF_HIP(hipMemcpy(ll.data(), fm->lo[fm->cur], fm->total * 4, hipMemcpyDeviceToHost));
+        } else {                // kept: behind the steps queued on the foam's stream
+            SF_HIP(hipMemcpyAsync(hh.data(), fm->hi[fm->cur_hi], fm->total * 4, hipMemcpyDeviceToHost, fm->stream));
+            SF_HIP(hipMemcpyAsync(ll.data(), fm->lo[fm->cur], fm->total * 4, hipMemcpyDeviceToHost, fm->stream));
         }
         if (gamma) {
             for (int64_t c = 0; c < fm->total; ++c) gg[c] = static_cast<float>(gamma[c]);
         } else {
-            SF_HIP(hipMemcpy(gg.data(), fm->g[fm->cur], fm->total * 4, hipMemcpyDeviceToHost));
+            SF_HIP(hipMemcpyAsync(gg.data(), fm->g[fm->cur], fm->total * 4, hipMemcpyDeviceToHost, fm->stream));
         }
+        SF_HIP(hipStreamSynchronize(fm->stream));
         fm->upload(hh.data(), ll.data(), gg.data());
         fm->resolve_cfl();
     });

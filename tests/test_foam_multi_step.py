@@ -110,3 +110,16 @@ def test_results_do_not_depend_on_the_active_set(name, grids, every):
     for a, b in zip(whole.fields(), some.fields()):
         for k in np.flatnonzero(mask):
             assert np.array_equal(whole.split(a)[k], some.split(b)[k]), (name, k)
+
+
+def test_kept_surfactant_waits_for_queued_steps():
+    """set_fields that keeps Γ right after queued steps: Γ as they leave it."""
+    grids = [(200 + 8 * k, 400 + 16 * k) for k in range(24)]
+    a, b = _foam(grids), _foam(grids)
+    h = np.full(a.length, 4e-7)
+    a.step(200)
+    a.set_fields(h)
+    b.step(200)
+    b.synchronize()
+    b.set_fields(h)
+    assert np.array_equal(a.fields()[1], b.fields()[1]) and np.array_equal(a.fields()[0], b.fields()[0])
