@@ -18,7 +18,10 @@
 //                             state, so forces read only the old positions
 //   cluster_contact_kernel    per (i, run): contacts j > i counted, the first
 //                             coalescence candidate in (i, j) order
-//   cluster_scan_kernel       one-block exclusive scan of the counts (i-major)
+//   cluster_offsets_kernel    offsets of the counts within each tile of 64
+//                             bubbles, in (i, run) order, and the tile's total
+//   cluster_tiles_kernel      the tiles' totals into first offsets, the first
+//                             candidate of all
 //   cluster_connect_kernel    BubbleConnection records written in (i, j) order
 //
 // Bubble state on the device: pr[i] = (x, y, z, radius), vt[i] = (vx, vy, vz,

@@ -87,3 +87,50 @@ def test_neighbors_of_other_ids(ids):
     sim.add_bubble((1.0, 1.0, 1.0), 0.01)
     R.add_bubble(c, (1.0, 1.0, 1.0), 0.01)
     assert sim.neighbors() == c.neighbors
+
+
+def _sparse_cluster(pairs, n=65600):
+    """n bubbles of 1 cm radius 10 cm apart on a lattice, and the second of
+    each pair moved to touch the first (21 mm between centres, within the
+    contact gap) on a side of its own."""
+    k = np.arange(n)
+    pos = 0.1 * np.stack([k % 41, k // 41 % 41, k // (41 * 41)], axis=1).astype(np.float64)
+    side = {}
+    for a, b in pairs:
+        d = np.zeros(3)
+        d[side.get(a, 0)] = 0.021
+        side[a] = side.get(a, 0) + 1
+        pos[b] = pos[a] + d
+    return pos, np.full(n, 0.01)
+
+
+# More than 1024 tiles of 64 bubbles: the tile totals are summed in rounds of
+# 1024 with a carry.  Contacts in the first and the second round and across,
+# several of one bubble, and the last bubble.
+PAIRS = [(5, 70), (5, 65537), (100, 65590), (31000, 31001), (65530, 65531), (65535, 65536), (65540, 65599),
+         (65545, 65546), (65545, 65550)]
+
+
+def test_contacts_past_1024_tiles():
+    pos, r = _sparse_cluster(PAIRS)
+    sim = _sim(pos, r)
+    assert [(x.bubble_a, x.bubble_b) for x in sim.connections()] == PAIRS
+    want = {}
+    for a, b in PAIRS:
+        want.setdefault(a, []).append(b)
+        want.setdefault(b, []).append(a)
+    assert {k: list(v) for k, v in enumerate(sim.neighbors()) if v} == want
+
+
+@pytest.mark.parametrize("fast", [[(65545, 65550)], [(65530, 65531), (65540, 65599)], [(65540, 65599), (100, 65590)]])
+def test_first_candidate_past_1024_tiles(fast):
+    """The connection that merges is the first in list order whose bubbles
+    close in fast enough, whichever round its tile is in."""
+    pos, r = _sparse_cluster(PAIRS)
+    vel = np.zeros_like(pos)
+    for a, b in fast:
+        vel[b] = 0.1 * np.sign(pos[a] - pos[b])        # 0.08 m/s after damping: a Weber number of 2.6
+    sim = _sim(pos, r, vel, coalescence_enabled=True, coalescence_threshold=1.0)
+    before = set(sim.bubbles()["ids"].tolist())
+    sim.step(1e-6)                                     # too short for the forces to move the others
+    assert before - set(sim.bubbles()["ids"].tolist()) == set(min(fast))
