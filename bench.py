@@ -287,7 +287,8 @@ def bench_foam(args, L, W):
     fm.step(max(1, args.warmup))
     fm.synchronize()
     fm.kernel_timing(True)
-    fm.step(min(args.steps, 200))
+    timed_steps = min(args.steps, 200)
+    fm.step(timed_steps)
     k_ms, k_n = fm.kernel_timing(False)
     fm.synchronize()
     t0 = time.perf_counter()
@@ -297,8 +298,15 @@ def bench_foam(args, L, W):
     info = fm.info()
     cells = info["cells"]
     st = fm.stats()
-    # With two steps per launch a timed launch advances every cell twice.
+    # With two steps per launch a timed launch advances every cell twice;
+    # small foams take several steps per launch by themselves.
     spl = fm.steps_per_launch()
+    multi = k_n > 0 and timed_steps / k_n > spl + 0.5
+    if multi:
+        spl = timed_steps / k_n
+    # the counters are those of 4096 bubbles on the streaming kernels
+    counted = len(bubbles) == 4096 and not multi
+    traffic, tsrc = pmc_traffic("c3" + ("-two-step" if spl == 2 else "")) if counted else (None, None)
     achieved = spl * BYTES_PER_CELL_STEP * cells / (k_ms * 1e-3) / 1e9
     out = {
         "metric": METRIC, "value": cells * args.steps / elapsed, "unit": "cell-steps/s",
@@ -308,7 +316,7 @@ def bench_foam(args, L, W):
         "config": {"workload": "foam of %d bubbles, n_theta ~ logU[32,512], n_phi = 2 n_theta, "
                                "diameter ~ logU[5,50] mm, h ~ U[200,1000] nm +-5 %%, viscosity ~ "
                                "U[1,5] mPa s, per-bubble CFL dt, Γ transport, 16-step HIP graphs, "
-                               "%d step(s) per launch" % (len(bubbles), spl),
+                               "%g step(s) per launch" % (len(bubbles), spl),
                    "bubbles": len(bubbles), "cells": cells, "items_per_launch": info["items"],
                    "steps_per_launch": spl,
                    "tile_shapes": info["variants"], "autotuned": chosen is not None,
@@ -316,9 +324,9 @@ def bench_foam(args, L, W):
                                                                      for row in trial]},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS,
-                     "traffic": pmc_traffic("c3" + ("-two-step" if spl == 2 else ""))[0],
-                     "traffic_source": traffic_source(pmc_traffic("c3" + ("-two-step" if spl == 2 else ""))[1]),
-                     "kernel": "foam_step2_kernel" if spl == 2 else "foam_step_kernel",
+                     "traffic": traffic, "traffic_source": traffic_source(tsrc),
+                     "kernel": ("foam_multi_kernel" if multi else
+                                "foam_step2_kernel" if spl == 2 else "foam_step_kernel"),
                      "steps_per_launch": spl,
                      "avg_launch_ms": k_ms, "launches_timed": k_n,
                      "algorithmic_bytes_per_launch": spl * BYTES_PER_CELL_STEP * cells},
@@ -654,7 +662,9 @@ def main():
         h0 = W.smooth_bubble(n_theta, n_phi, seed=3)
         flags = L.FLAG_TFE | L.FLAG_SURFACTANT | L.FLAG_DIAG
         desc = ("single bubble %dx%d FP32 drainage, CFL dt" % (n_theta, n_phi)
-                + (" + 81-wavelength spectral RGB per step (FP16 MFMA, FP32 accumulate)" if spectral else ""))
+                + (" + 81-wavelength spectral RGB per step (%s)"
+                   % ("FP32 cosine series, FP16 MFMA near grazing" if n_theta * n_phi >= SPECTRAL_SERIES_CELLS
+                      else "FP16 MFMA, FP32 accumulate") if spectral else ""))
     if args.flags is not None:
         flags = args.flags
     p = L.Params()
