@@ -133,18 +133,53 @@ __global__ __launch_bounds__(256) void gemm_kernel(const GemmArgs g) {
 
 // ---- elementwise -------------------------------------------------------------
 
-__device__ inline float gelu(float z) {      // tanh form
+// GELU (tanh form), 0.5 z (1 + tanh u) with u = k0 (z + k1 z^3), and its
+// derivative, in FP32 throughout.  Up to |z| = kGeluSmall tanh is a polynomial
+// (minimax on |u| <= 0.4, 2e-9 relative); past it both come from
+// e = exp(-2 |u|) <= 1, so that neither 1 + tanh nor 1 - tanh^2 cancels:
+//   gelu = max(z, 0) - |z| e / (1 + e),
+//   gelu' = g for z < 0 and 1 - g for z > 0, g = (1 - 2 |z| u' / (1 + e)) e / (1 + e).
+// 2-norm errors over z ~ N(0, 1) 3.0e-8 and 3.6e-8 (with tanhf 3.7e-8 and
+// 4.5e-8), over N(0, 0.1^2) 2.7e-8 and 2.9e-8 (3.8e-8, 3.9e-8), over N(0, 3^2)
+// 2.1e-8 and 3.6e-8 (2.8e-8, 1.4e-7).
+constexpr float kGeluSmall = 0.49f;
+
+struct GeluTerms {
+    float t, du, s, es;      // tanh u (small z), u', 1 / (1 + e), e / (1 + e)
+};
+
+__device__ inline GeluTerms gelu_terms(float z) {
     const float k0 = 0.7978845608028654f, k1 = 0.044715f;
-    return 0.5f * z * (1.f + tanhf(k0 * (z + k1 * z * z * z)));
+    const float z2 = z * z;
+    const float u = k0 * z * fmaf(k1, z2, 1.f), w = u * u;
+    GeluTerms g;
+    g.t = fmaf(u * w, fmaf(fmaf(fmaf(0.01874406f, w, -0.053561937f), w, 0.13331214f), w, -0.333333f), u);
+    g.du = k0 * fmaf(3.f * k1, z2, 1.f);
+    const float e = __builtin_amdgcn_exp2f(-2.8853900817779268f * fabsf(u));
+    g.s = __builtin_amdgcn_rcpf(1.f + e);
+    g.es = e * g.s;
+    return g;
+}
+
+__device__ inline float gelu(float z) {
+    const GeluTerms g = gelu_terms(z);
+    const float a = fabsf(z), v = 0.5f * z;
+    // the product is zero, not a NaN, at infinity
+    return a < kGeluSmall ? fmaf(v, g.t, v) : fmaxf(z, 0.f) - fminf(a, 3e38f) * g.es;
+}
+
+__device__ inline float gelu_grad(float z) {
+    const GeluTerms g = gelu_terms(z);
+    const float q = z * g.du;
+    const float h = g.es * fmaf(-2.f * fabsf(q), g.s, 1.f);
+    if (fabsf(z) < kGeluSmall) return fmaf(0.5f, fmaf(q, fmaf(-g.t, g.t, 1.f), g.t), 0.5f);
+    return z > 0.f ? 1.f - h : h;
 }
 
 __device__ inline float gelu_exp(float z) {
     // 0.5 z (1 + tanh u) = z / (1 + exp(-2u)), u = k0 (z + k1 z^3); hardware
     // exp2 and reciprocal (about 1e-6 relative, far below the BF16 rounding
-    // the result is stored with: inference only.  Training, which stores
-    // FP32, takes gelu and gelu_grad: 2-norm errors over z ~ N(0, 1) 3.7e-8
-    // and 4.5e-8 against 4.7e-8 and 7.4e-8 in this form, over N(0, 3^2) of
-    // the derivative 1.4e-7 against 3.6e-7)
+    // the result is stored with: inference in 16 bits only)
     const float k0 = 0.7978845608028654f, k1 = 0.044715f;
     const float u = k0 * fmaf(k1 * z, z * z, z);
     const float e = __builtin_amdgcn_exp2f(-2.8853900817779268f * u);
@@ -580,13 +615,6 @@ __global__ __launch_bounds__(256) void fno_row_wave_kernel(const RowArgs a, int 
     }
 }
 
-__device__ inline float gelu_grad(float z) {
-    const float k0 = 0.7978845608028654f, k1 = 0.044715f;
-    const float u = k0 * (z + k1 * z * z * z);
-    const float t = tanhf(u);
-    return 0.5f * (1.f + t) + 0.5f * z * (1.f - t * t) * k0 * (1.f + 3.f * k1 * z * z);
-}
-
 // x_out = act(z), z = z_in + bias[c] (+ y), over n rows of C channels.
 __global__ void bias_act_kernel(float* z, const float* y, const float* bias, float* x_out, long long total, int C,
                                 int act) {
@@ -921,9 +949,9 @@ __global__ __launch_bounds__(256) void column_partial_kernel(const float* x, lon
 // compensated FP32 of the unrounded values.
 //
 // What bounds it: 512 B per cell (dz, z, x in, dz out) of HBM traffic, 200 us
-// at 5.4 TB/s for 16 bubbles of 256 x 512 at width 32; measured 313 us (3.4
-// TB/s, latency: 128 registers allow four waves per SIMD; 428 us with one
-// block per CU).  It replaces, per layer, act_grad (148 us), three passes for
+// at 5.4 TB/s for 16 bubbles of 256 x 512 at width 32; measured 322-330 us (3.3
+// TB/s, latency: 128 registers allow four waves per SIMD; a third more with
+// one block per CU).  It replaces, per layer, act_grad (148 us), three passes for
 // the bias and weight gradients (183 + 18 + 300 us) and three row GEMMs of 300
 // us each: a training window's backward pass went from 7.5 to 1.6 ms.
 constexpr int kBackUnroll = 1;
