@@ -419,9 +419,13 @@ int sf_foam_use_graph(sf_foam* foam, int32_t enable);
  * two-step kernel's halo columns), so both give identical results.  Small
  * foams (rows of at most 1024 columns, up to 2 blocks of at most 16 rows per
  * compute unit) take up to 8 steps per launch by themselves, with pole means
- * from FP64 ring sums; a call here, or explicit tile shapes, switches that
- * off.  No counterpart
- * in the reference (foam.rs keeps no per-bubble grids). */
+ * from FP64 ring sums; the foam's whole size decides, held bubbles included,
+ * so that results do not depend on the set of active bubbles or on how steps
+ * are grouped into calls.  A call here, also with the value got before, or
+ * explicit tile shapes put the foam on the streaming kernels for the rest of
+ * its life (pole means agree to the last bits).  The value got is the
+ * streaming kernels'; what a small foam takes by itself is not counted in.
+ * No counterpart in the reference (foam.rs keeps no per-bubble grids). */
 int sf_foam_set_steps_per_launch(sf_foam* foam, int32_t steps);
 int sf_foam_get_steps_per_launch(sf_foam* foam, int32_t* steps);
 /* Tile shapes: a wave streams a band of rows of one column chunk.
@@ -434,7 +438,9 @@ int sf_foam_get_steps_per_launch(sf_foam* foam, int32_t* steps);
  * <= 384, > 384) for trial_steps steps on a copy of the state, keeps the
  * fastest per bucket and restores the state.  chosen[4] receives the shape
  * per bucket, trial_ms[4][10] the average kernel time per step of each trial (-1
- * for buckets without bubbles or shapes not tried); either may be NULL. */
+ * for buckets without bubbles or shapes not tried); either may be NULL.  Small
+ * foams that take several steps per launch by themselves use the shapes only
+ * after sf_foam_set_steps_per_launch. */
 int sf_foam_autotune(sf_foam* foam, int32_t trial_steps, int32_t* chosen, double* trial_ms);
 /* Sets the tile shape index (0-9, as above) of each of the 4 buckets. */
 int sf_foam_set_tile_shapes(sf_foam* foam, const int32_t* shapes);

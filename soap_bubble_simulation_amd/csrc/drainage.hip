@@ -491,9 +491,9 @@ void Drainage::upload_tables() {
     tables_dirty = false;
 }
 
-// FP64 pole-row film volume, used while the h poles are copied through.
-// The pole rows' film volume, added up on the host in column order, and the
-// largest thickness where the last split left its maxima.
+// FP64 film volume of the pole rows, added up on the host in column order
+// (used while they are copied through), and the largest thickness where the
+// last split left its maxima.
 void Drainage::update_fixed_pole_mass(bool with_max) {
     const size_t w = static_cast<size_t>(np);
     hipLaunchKernelGGL(pole_rows_kernel, dim3(std::min<unsigned>(cdiv(4 * w, 256), 256)), dim3(256), 0, stream,

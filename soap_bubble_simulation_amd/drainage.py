@@ -166,11 +166,15 @@ class DrainageContext:
 
     def set_steps_per_launch(self, steps: int) -> None:
         """1, or 2 for two steps per stencil launch where the flags and grid
-        allow it (bit-identical results; see ``steps_per_launch``)."""
+        allow it (bit-identical to each other; see ``steps_per_launch``).
+        Small grids take up to 8 steps per launch by themselves; a call here,
+        also with the value ``steps_per_launch`` returns, puts them on the
+        streaming kernels for good (same fields to FP32 rounding)."""
         L.check(self._lib.sf_drainage_set_steps_per_launch(self._h, int(steps)))
 
     def steps_per_launch(self) -> int:
-        """Steps per stencil launch that ``step`` uses for this context."""
+        """Steps per launch, 1 or 2, of the streaming kernels for this
+        context (what a small grid takes by itself is not counted in)."""
         k = C.c_int32()
         L.check(self._lib.sf_drainage_get_steps_per_launch(self._h, C.byref(k)))
         return k.value

@@ -130,7 +130,9 @@ class FoamDrainage:
 
     def set_steps_per_launch(self, steps: int) -> None:
         """1 or 2 steps per stencil launch (two: the state is streamed once
-        per two steps, bit-identical to one-step launches)."""
+        per two steps, bit-identical to one-step launches).  Small foams take
+        up to 8 steps per launch by themselves; a call here puts them on the
+        streaming kernels for good (pole means to the last bits)."""
         L.check(self._lib.sf_foam_set_steps_per_launch(self._h, int(steps)))
 
     def steps_per_launch(self) -> int:
@@ -140,7 +142,9 @@ class FoamDrainage:
 
     def autotune(self, trial_steps: int = 8, return_times: bool = False):
         """Picks the fastest tile shape per size bucket; optionally also
-        returns the trial kernel times [bucket][shape] in ms (-1: empty)."""
+        returns the trial kernel times [bucket][shape] in ms (-1: empty).
+        Small foams, which take several steps per launch by themselves, use
+        the shapes only after ``set_steps_per_launch``."""
         chosen = (C.c_int32 * 4)()
         times = np.empty(4 * len(TILE_SHAPES), np.float64)
         L.check(self._lib.sf_foam_autotune(self._h, int(trial_steps), chosen, L.dptr(times)))
