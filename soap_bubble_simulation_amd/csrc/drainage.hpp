@@ -149,7 +149,7 @@ struct Drainage {
     int cmf_skip = 0;               // trailing wavelength slots the spectral pass leaves out
     int spec_operand = 0;           // SF_SPECTRAL_OPERAND_*
     float4* spec_rows = nullptr;
-    float2* spec_view = nullptr;    // per-cell (q, opd per thickness) of spec_view_key's camera and index
+    float2* spec_view = nullptr;    // per-cell (q or F, opd per thickness) of spec_view_key's camera and index
     float spec_view_key[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     bool spec_view_valid = false;
     float2* spec_cols = nullptr;

@@ -3,8 +3,8 @@
 ``InterferenceCalculator`` mirrors src/physics/interference.rs:127-513 and
 ``generate_interference_lut`` mirrors src/render/interference_lut.rs:18-41.
 Every evaluation, including the single-point helpers, runs in a HIP kernel
-(FP32 arithmetic); LUT addressing is formed on the host in FP64 exactly like
-the reference.
+(FP32 arithmetic); LUT addressing is formed there in FP64 exactly like the
+reference.
 """
 from __future__ import annotations
 
