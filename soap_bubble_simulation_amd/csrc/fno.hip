@@ -740,8 +740,10 @@ struct Fno {
     }
 
     // Inference keeps activations between layers in 16 bits at n_phi 512 and
-    // 128.  n_phi = 256 runs the training pass's kernels instead: activations
-    // in FP32 and the lift formed in FP32, which its outputs always had.
+    // 128.  n_phi = 256 runs the training pass's layer kernels instead:
+    // activations in FP32 and the lift formed in FP32, which its outputs
+    // always had (8 bubbles of 128 x 256, two windows: 0.75 ms; the 16-bit
+    // kernels took 0.76-0.78, the batched GEMMs 1.6).
     bool inference16() const { return P != 256; }
 
     // Kernel paths the forward passes take at this shape (SF_FNO_PATH_* bits).
@@ -751,7 +753,7 @@ struct Fno {
             p |= SF_FNO_PATH_FUSED_ROWS;
             if (static_cast<size_t>(P * kCin + 2 * Mp * (kCin + 1)) * sizeof(float) <= 64 * 1024 && P <= kLiftDftMaxP)
                 p |= SF_FNO_PATH_LIFT_DFT;
-            if (inference16() && theta_fused_ok()) p |= SF_FNO_PATH_FUSED_THETA;
+            if (theta_fused_ok()) p |= SF_FNO_PATH_FUSED_THETA;
             if (inference16() && row_wave_kernel()) p |= SF_FNO_PATH_WAVE_ROWS;
         }
         return p;
@@ -836,7 +838,10 @@ struct Fno {
             // output in FP32 and, for the backward pass, its pre-activations.
             lift_dft(B);
             for (int l = 0; l < L; ++l) {
-                theta_stage(l, B);
+                if (training)
+                    theta_stage(l, B);       // keeps the spectrum
+                else
+                    theta_stage_inference(l, B);
                 const bool last = l == L - 1;
                 RowArgs ra{xs[l], Z, w + o_w[l], w + o_b[l], Iphi16, Ephi16, xs[l + 1], training ? zs[l] : nullptr,
                            last ? nullptr : X1, last ? 0 : 1, l == 0 ? in : nullptr, w + o_wl, w + o_bl, w + o_q, w + o_qb,

@@ -232,7 +232,7 @@ def test_gpu_inference_at_256_columns_keeps_fp32(width, modes_phi, layers):
     from soap_bubble_simulation_amd.surrogate import FnoSurrogate
     m = FnoSurrogate(n_theta=32, n_phi=256, width=width, modes_theta=8, modes_phi=modes_phi, layers=layers, window=4,
                      max_batch=2)
-    assert m.kernel_paths() == L.FNO_PATH_FUSED_ROWS | L.FNO_PATH_LIFT_DFT
+    assert m.kernel_paths() == L.FNO_PATH_FUSED_ROWS | L.FNO_PATH_LIFT_DFT | L.FNO_PATH_FUSED_THETA
     s = R.Shapes.of(m.config)
     flat, x, _ = rand_problem(s, 2, seed=12, scale=0.25)
     f32, x32 = flat.astype(np.float32), x.astype(np.float32)
